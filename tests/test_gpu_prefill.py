@@ -224,6 +224,47 @@ def test_prefill_large_grid_paged_cached_prefix_subtiles(B, lq, cached, Hq, Hkv,
         assert bool((err <= ATOL + RTOL * ref.abs()).all()), f"sequence {b}: worst {err.max().item():.4g}"
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,B,BS,scale", [
+    (12, 4, 64, 5, 0, 0.125),      # two row tiles of a kv head's XCD pair
+    (15, 3, 64, 4, 48, 0.2),       # kv heads that do not divide 8, G = 5, blocks of 48
+    (7, 1, 128, 3, 16, -0.1),      # one kv head over 8 XCDs, G = 7, a negative scale
+    (16, 16, 64, 6, 32, 0.0),      # more kv heads than XCDs, equal weights
+    (32, 8, 128, 64, 64, 0.09),    # as many sequences as lanes rank
+    (32, 8, 128, 65, 0, 0.09),     # one more: tiles in index order
+])
+def test_prefill_ragged_work_items(Hq, Hkv, D, B, BS, scale):
+    """Every (sequence, 128-row tile, kv head) is computed once whatever the
+    order of the work: ragged lengths around the 64-key and 128-row edges,
+    empty sequences, cached prefixes, and a max_seqlen_q above the longest.
+    Bound as above (weights and output rounded to bf16)."""
+    rng = np.random.default_rng(B + D + BS)
+    G = Hq // Hkv
+    edge = 128 // G
+    pool = [0, 1, edge - 1, edge, edge + 1, 63, 64, 65, 128, 129, 2 * edge + 1, 200]
+    lens_k = np.array([pool[(3 * b + 11) % 12] if b % 7 else 200 for b in range(B)])
+    lens_q = np.array([n if BS == 0 or b % 3 == 0 else -(-n // (b % 3 + 1)) for b, n in enumerate(lens_k)])
+    cu_q, cu_k = (torch.tensor(np.concatenate([[0], np.cumsum(n)]), dtype=torch.int32, device=DEV)
+                  for n in (lens_q, lens_k))
+    q = bf16(rng, int(lens_q.sum()), Hq, D)
+    kw, bt = {}, None
+    if BS:
+        nblk = -(-lens_k // BS)
+        perm = rng.permutation(int(nblk.sum()) + 2)
+        bt = np.full((B, int(nblk.max()) + 1), -1, np.int32)
+        at = 0
+        for b, n in enumerate(nblk):
+            bt[b, :n] = perm[at:at + n]
+            at += n
+        k, v = (bf16(rng, len(perm), BS, Hkv, D) for _ in range(2))
+        kw = dict(block_table=torch.from_numpy(bt).to(DEV))
+    else:
+        k, v = (bf16(rng, int(lens_k.sum()), Hkv, D) for _ in range(2))
+    o = K.flash_attn_varlen_func(q, k, v, cu_q, cu_k, int(lens_q.max()) + 70, int(lens_k.max()), scale, **kw)
+    ref = P.prefill_attention(f64(q), f64(k), f64(v), cu_q.cpu().numpy(), cu_k.cpu().numpy(), scale,
+                              **({"block_tables": bt} if BS else {}))
+    assert_close(f64(o), ref, f"work items Hq={Hq} Hkv={Hkv} D={D} B={B} BS={BS}")
+
+
 def test_prefill_argument_errors():
     q = torch.zeros(4, 8, 64, dtype=torch.bfloat16, device=DEV)
     kv = torch.zeros(4, 2, 64, dtype=torch.bfloat16, device=DEV)
