@@ -341,6 +341,11 @@ struct DecodeWave {
 struct NoPrologue {
   __device__ __forceinline__ void operator()() const {}
 };
+// t / BS for t >= 0, by a 32-bit divide where t < 2^31 (every real pool)
+__device__ __forceinline__ int64_t block_of(int64_t t, int BS) {
+  return t >> 31 ? t / BS : (int64_t)((unsigned)t / (unsigned)BS);
+}
+
 template <int D, int G, class Pro = NoPrologue>
 __device__ __forceinline__ void decode_walk(
     DecodeWave<D, G>& w, const typename DecodeWave<D, G>::QBuf& qa, const uint16_t* __restrict__ kc,
@@ -350,7 +355,7 @@ __device__ __forceinline__ void decode_walk(
   using W = DecodeWave<D, G>;
   const int lane = w.lane;
   const int64_t step_rows = (int64_t)tile * tstride;
-  const int ntiles = (int)((t_end - t_begin + step_rows - 1) / step_rows);
+  const int ntiles = (int)block_of(t_end - t_begin + step_rows - 1, (int)step_rows);
   // The walk's block ids, 256 at a time (window w0 .. w0 + 255 of the table
   // row): lane l holds ids 4l .. 4l+3 of the window, read back with
   // readlane, so no tile waits on a scalar load of its block id.  Ids at or
@@ -359,7 +364,7 @@ __device__ __forceinline__ void decode_walk(
   // there: the group's tiles then read ids with no load pending on them, so
   // the compiler puts no vmcnt(0) between a tile's loads and the next
   // tile's (which would drain the tile in flight).  A group spans
-  // (MAXT-1)*tstride*tile + tile <= 256*BS rows for tstride <= 36.
+  // (MAXT-1)*(tstride*tile/BS + 1) + 1 <= 256 blocks for tstride <= 35.
   int64_t w0 = -1;
   uint4 ids = make_uint4(0, 0, 0, 0);
   auto load_window = [&](int64_t wb) {
@@ -381,19 +386,29 @@ __device__ __forceinline__ void decode_walk(
   // element offset of its first row.  Tiles at or past `last` are
   // look-ahead fillers: n = 0 and row 0 of block 0, so their loads all hit
   // one line (they only keep the per-step load count constant).
+  // The tiles are asked for in order, so the block column and the row within
+  // the block of the next one are carried along: a divide per tile (64-bit,
+  // some 100 instructions) would sit between a tile's arithmetic and the next
+  // tile's loads.
   int last = 0;
+  const int sq = (int)step_rows / BS, sr = (int)step_rows - sq * BS;
+  int64_t left = t_end - t_begin, bi = block_of(t_begin, BS);
+  int bo = (int)(t_begin - bi * BS);
   auto tile_at = [&](int i, int& n, int64_t& off) {
     if (i >= last) {
       n = 0;
       off = (int64_t)kh * D;
       return;
     }
-    const int64_t t0 = t_begin + (int64_t)i * step_rows;
-    n = (int)min((int64_t)tile, t_end - t0);
-    const int32_t blk = block_id(t0 / BS);
+    n = (int)min((int64_t)tile, left);
+    const int32_t blk = block_id(bi);
     const bool ok = blk >= 0 && (int64_t)blk < NB;
     if (!ok) n = 0;  // invalid block: contributes nothing
-    off = ((int64_t)(ok ? blk : 0) * BS + (t0 % BS)) * w.row + (int64_t)kh * D;
+    off = ((int64_t)(ok ? blk : 0) * BS + bo) * w.row + (int64_t)kh * D;
+    left -= step_rows;
+    bi += sq;
+    bo += sr;
+    if (bo >= BS) bo -= BS, ++bi;
   };
 
   // Pipeline one tile deep over two K and two V buffers: step i issues the
@@ -421,9 +436,8 @@ __device__ __forceinline__ void decode_walk(
   for (int base = 0; base < ntiles; base += MAXT) {
     last = min(ntiles, base + MAXT);
     {
-      const int64_t bf = (t_begin + (int64_t)base * step_rows) / BS;
-      const int64_t bl = (t_begin + (int64_t)(last - 1) * step_rows) / BS;
-      if (base == 0 || __builtin_amdgcn_readfirstlane((int)(bf < w0 || bl >= w0 + 256))) load_window(bf);
+      const int64_t bl = bi + (last - 1 - base) * (sq + 1);  // no tile of the group lies past it
+      if (base == 0 || __builtin_amdgcn_readfirstlane((int)(bl >= w0 + 256))) load_window(bi);
     }
     {
       int64_t o0;
@@ -463,7 +477,7 @@ __device__ __forceinline__ void decode_chunk(
   typename W::QBuf qa;
   w.load_q(qa, q, b, kh, Hq);
   decode_walk<D, G>(w, qa, kc, vc, btrow, BS, NB, tile, scale_log2, kh, t_begin, t_end, 1,
-                    (t_end - 1) / BS + 1, pw);
+                    block_of(t_end - 1, BS) + 1, pw);
   w.finish(t_begin == 0 && t_end >= Lc, out, ws_o, ws_ml, b, kh, Hq, prow);
 }
 
@@ -520,7 +534,7 @@ constexpr int BAL_MAXB = 8192;
 
 __device__ __forceinline__ int decode_tiles(const int64_t* ctx_lens, int b, int64_t cap, int tile) {
   const int64_t L = min(ctx_lens[b], cap);
-  return L > 0 ? (int)((L + tile - 1) / tile) : 0;
+  return L > 0 ? (int)((L + tile - 1) >> __builtin_ctz(tile)) : 0;  // tile is 16, 32 or 64
 }
 
 template <int D, int G>
@@ -563,38 +577,40 @@ __global__ __launch_bounds__(256) void paged_decode_balanced(
   if (blockIdx.x == 0)
     for (int i = tid; i <= B; i += nthr) tp_out[i] = tp[i];
 
-  const int64_t total = (int64_t)ngroups * tp[B];
-  const int nwg = gridDim.x;
-  const int64_t Ct = max((int64_t)1, (total + nwg - 1) / nwg);
-  int64_t u = (int64_t)blockIdx.x * Ct;
-  const int64_t u_end = min(total, u + Ct);
+  // 32-bit throughout: the host refuses 2^31 work units, and a 64-bit divide
+  // is some 0.3 us of a chain that no other work hides
+  const unsigned total = (unsigned)ngroups * (unsigned)tp[B];
+  const unsigned nwg = gridDim.x;
+  const unsigned Ct = max(1u, (total + nwg - 1) / nwg);
+  unsigned u = blockIdx.x * Ct;
+  const unsigned u_end = min(total, u + Ct);
   if (u >= u_end) return;
   // first sequence: the largest b with ngroups * tp[b] <= u (it has n_b > 0)
   int b_lo = 0, b_hi = B - 1;
   while (b_lo < b_hi) {
     const int mid = (b_lo + b_hi + 1) >> 1;
-    if ((int64_t)ngroups * tp[mid] <= u) b_lo = mid;
+    if ((unsigned)ngroups * (unsigned)tp[mid] <= u) b_lo = mid;
     else b_hi = mid - 1;
   }
   int b = b_lo;
   float* pw = p_lds[wave];
   while (u < u_end) {
-    const int nb = tp[b + 1] - tp[b];
-    const int64_t base = (int64_t)ngroups * tp[b];
+    const unsigned nb = tp[b + 1] - tp[b];
+    const unsigned base = (unsigned)ngroups * (unsigned)tp[b];
     const int grp = (int)((u - base) / nb);
-    const int64_t i0 = (u - base) - (int64_t)grp * nb;
-    const int64_t seg_end = min(u_end, base + (int64_t)(grp + 1) * nb);
+    const unsigned i0 = (u - base) - grp * nb;
+    const unsigned seg_end = min(u_end, base + (grp + 1) * nb);
     const int kh = grp * wpg + wave;
     if (kh < Hkv) {
       const int64_t Lc = min(ctx_lens[b], cap);
-      const int64_t t_begin = i0 * tile;
-      const int64_t t_end = min(Lc, (i0 + (seg_end - u)) * tile);
+      const int64_t t_begin = (int64_t)i0 * tile;
+      const int64_t t_end = min(Lc, (int64_t)(i0 + (seg_end - u)) * tile);
       const int64_t slot = ((int64_t)blockIdx.x + (int64_t)b * ngroups + grp) * wpg + wave;
       decode_chunk<D, G>(q, kc, vc, bt + (int64_t)b * bt_stride, ws_o, ws_ml, out, Hkv, BS, NB, tile,
                          scale_log2, b, kh, t_begin, t_end, Lc, slot * G, pw, lane);
     }
     u = seg_end;
-    if (u >= base + (int64_t)ngroups * nb) {
+    if (u >= base + ngroups * nb) {
       ++b;
       while (b < B && tp[b + 1] == tp[b]) ++b;  // sequences with no context
     }
@@ -892,18 +908,24 @@ __device__ __forceinline__ int part_span(const PartMap& pm, int b, int h, int Hq
   if (nb == 0) return 0;
   const int kh = h / pm.G, g = h - kh * pm.G;
   const int grp = kh / pm.wpg, wv = kh - grp * pm.wpg;
-  const int64_t total = (int64_t)pm.ngroups * pm.tp[pm.B];
-  const int64_t Ct = max((int64_t)1, (total + pm.nwg - 1) / pm.nwg);
-  const int64_t start = (int64_t)pm.ngroups * pm.tp[b] + (int64_t)grp * nb;
-  const int64_t wf = start / Ct, wl = (start + nb - 1) / Ct;
-  r0 = ((wf + (int64_t)b * pm.ngroups + grp) * pm.wpg + wv) * pm.G + g;
+  const unsigned total = (unsigned)pm.ngroups * (unsigned)pm.tp[pm.B];  // < 2^31, as in the split
+  const unsigned Ct = max(1u, (total + pm.nwg - 1) / (unsigned)pm.nwg);
+  const unsigned start = (unsigned)pm.ngroups * (unsigned)pm.tp[b] + (unsigned)grp * (unsigned)nb;
+  const unsigned wf = start / Ct, wl = (start + nb - 1) / Ct;
+  r0 = (((int64_t)wf + (int64_t)b * pm.ngroups + grp) * pm.wpg + wv) * pm.G + g;
   return (int)(wl - wf + 1);
 }
 
 // Log-sum-exp merge of one output element: partials s = 0 .. ns-1 of a
-// (sequence, head) at workspace rows r0 + s*rs, element d.  Up to MERGE_NS
-// partials are loaded together (one memory round trip), more in a loop with
-// the same arithmetic in the same order.  ns == 0 (no context) gives 0.
+// (sequence, head) at workspace rows r0 + s*rs, element d.  All lanes of a
+// wave share the (sequence, head) (D is a multiple of 64).  Up to MERGE_NS
+// partials are loaded together (one memory round trip).  More (a few long
+// contexts spread over the whole chip) go 64 at a time: lane s loads the
+// (m, l) and computes the weight of partial s, while every lane's 64 values
+// are already in flight; the sums take the weights by readlane in the same
+// order as before, so the same bits.  Measured at three sequences of 583-2517
+// tokens (40-69 partials a row): 28.1 -> 6.9 us against a loop of one partial
+// at a time, which waits a round trip for each.  ns == 0 (no context) gives 0.
 constexpr int MERGE_NS = 16;
 __device__ __forceinline__ float merge_element(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
                                                int64_t r0, int64_t rs, int ns, int D, int d) {
@@ -933,16 +955,27 @@ __device__ __forceinline__ float merge_element(const float* __restrict__ ws_o, c
     }
     res = den > 0.f ? num / den : 0.f;
   } else if (ns > 1) {
-    float M = -INFINITY;
-    for (int s = 0; s < ns; ++s) M = fmaxf(M, ws_ml[(r0 + s * rs) * 2]);
-    float num = 0.f, den = 0.f;
-    if (M != -INFINITY) {
-      for (int s = 0; s < ns; ++s) {
-        const int64_t r = r0 + s * rs;
-        const float w = exp2f(ws_ml[r * 2] - M);
-        den = fmaf(w, ws_ml[r * 2 + 1], den);
-        num = fmaf(w, ws_o[r * D + d], num);
-      }
+    const int lane = threadIdx.x & 63;
+    float M = -INFINITY, num = 0.f, den = 0.f;
+    for (int c = 64; c < ns; c += 64)  // the chunks past the first, whose maximum comes with its values
+      M = fmaxf(M, ws_ml[(r0 + min(c + lane, ns - 1) * rs) * 2]);
+    for (int c = 0; c < ns; c += 64) {
+      const int n = min(64, ns - c);
+      const int64_t r = r0 + c * rs;
+      const float m = ws_ml[(r + min(lane, n - 1) * rs) * 2], l = ws_ml[(r + min(lane, n - 1) * rs) * 2 + 1];
+      float ov[64];
+#pragma unroll
+      for (int s = 0; s < 64; ++s) ov[s] = ws_o[(r + min(s, n - 1) * rs) * D + d];
+      if (c == 0) M = group_max<64>(fmaxf(M, m));
+      if (M == -INFINITY) break;
+      const float w = exp2f(m - M);
+#pragma unroll
+      for (int s = 0; s < 64; ++s)
+        if (s < n) {
+          const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), s));
+          den = fmaf(ws, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l), s)), den);
+          num = fmaf(ws, ov[s], num);
+        }
     }
     res = den > 0.f ? num / den : 0.f;
   }

@@ -530,3 +530,41 @@ def test_decode_step_store_then_attend():
     qh, kh, vh, bth = host_inputs(case, kc, vc, q)
     assert_close(o.float().cpu().numpy(), P.paged_decode(qh, kh, vh, case.context_lens, bth, case.scale),
                  "store+decode")
+
+
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,D,BS,lens", [
+    (32, 8, 128, 16, [270, 0, 271, 1]),       # 17 partials a row and fewer: the edge of the one-trip merge
+    (16, 4, 64, 16, [4096]),                  # 256 partials a row: several chunks of 64
+    (32, 8, 128, 48, [1040, 1050, 30]),       # blocks that are no power of two, 64 and more partials
+    (12, 4, 64, 64, [63, 64, 65, 5000]),
+])
+def test_decode_many_partials_per_row(Hq, Hkv, D, BS, lens, quant):
+    """Few long contexts spread over the whole chip: rows of 17 to 256
+    partials through the merge, against the float64 oracle and (to fp32
+    summation order, so a bf16 rounding) the fixed chunks of one block."""
+    rng = np.random.default_rng(Hq + BS + len(lens))
+    lens = np.array(lens, np.int64)
+    nblk = -(-lens // BS)
+    perm = rng.permutation(int(nblk.sum()) + 3)
+    bt = np.full((len(lens), int(nblk.max())), -1, np.int32)
+    at = 0
+    for b, n in enumerate(nblk):
+        bt[b, :n] = perm[at:at + n]
+        at += n
+    g = torch.Generator(device="cuda").manual_seed(BS)
+    kc, vc = (torch.randn(len(perm), BS, Hkv, D, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(len(lens), Hq, D, generator=g, device="cuda").to(torch.bfloat16)
+    args = (q, kc, vc, torch.from_numpy(lens).cuda(), torch.from_numpy(bt).cuda())
+    res = K.paged_attention_decode(*args, blocks_per_split=0, quant=quant)
+    o = res[0] if quant else res
+    one = K.paged_attention_decode(*args, blocks_per_split=1)
+    ref = P.paged_decode(q.double().cpu().numpy(), kc.double().cpu().numpy(), vc.double().cpu().numpy(), lens, bt,
+                         D ** -0.5)
+    err = np.abs(o.double().cpu().numpy() - ref)
+    assert (err <= 2e-2 + 1e-2 * np.abs(ref)).all(), err.max()
+    # one bf16 rounding apart at most: 2^-8 of the value
+    assert bool(((o.float() - one.float()).abs() <= 2.0 ** -7 * one.float().abs() + 1e-6).all())
+    if quant:
+        codes, scales = K.act_quant(o.reshape(len(lens), -1))
+        assert torch.equal(res[1].view(torch.uint8), codes.view(torch.uint8)) and torch.equal(res[2], scales)
