@@ -28,6 +28,9 @@
 // bf16.  Row reductions (the RMS mean, the gate dot products) are summed in a
 // different order than torch's reduction kernels, so their results can differ
 // in the last fp32 bit.
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 #include "rope.h"
 
@@ -394,6 +397,113 @@ __global__ __launch_bounds__(64 * kRouteTokens) void moe_route_kernel(
   }
 }
 
+// Large batches in index form (the grouped dispatch: no routed bias), E <= EP
+// = 8, 16 or 32 experts: a wave takes 32 / EP tokens, so that each gate row
+// chunk is unpacked once for them and the tokens' memory round trips overlap.
+// Their 32 logits are summed by halving: at lane distance 32, 16, 8, 4, 2 a
+// lane hands half of its sums over and keeps the others, the pairs and order
+// of the butterfly (the same bits) in 31 additions instead of 192, and
+// lane bits 5..1 end as (token, expert).  Each group of 2 * EP lanes then
+// picks its token's top k.  16384 tokens, d 768, 8 experts: 39 -> 13 us
+// against a wave per token, which waits out its loads, its eight butterflies
+// and its picks one after the other.
+template <int O>
+__device__ __forceinline__ float halve(float a, float b) {  // lane & O ? b(lane ^ O) + b : a + a(lane ^ O)
+  if constexpr (O == 32 || O == 16) {
+    const auto r = O == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_int(a), __float_as_int(b), false, false)
+                           : __builtin_amdgcn_permlane16_swap(__float_as_int(a), __float_as_int(b), false, false);
+    return as_float((int)r[0]) + as_float((int)r[1]);
+  } else {
+    const bool up = __lane_id() & O;
+    const float give = up ? a : b, keep = up ? b : a;
+    return keep + as_float(xor_partner<O>(__float_as_int(give)));
+  }
+}
+
+template <int EP>
+__global__ __launch_bounds__(256) void moe_route_rows_kernel(const uint16_t* __restrict__ h,
+                                                             const uint16_t* __restrict__ gw,
+                                                             const float* __restrict__ ebias,
+                                                             float* __restrict__ dense, int64_t T, int d, int E, int S,
+                                                             int top_k, int64_t* __restrict__ topk_idx,
+                                                             float* __restrict__ topk_w) {
+  constexpr int TW = 32 / EP;  // tokens per wave
+  const int lane = threadIdx.x & 63;
+  const int64_t t0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * TW;
+  if (t0 >= T) return;
+  const int cpr = d / 8;
+  float acc[32];  // token, expert
+#pragma unroll
+  for (int x = 0; x < 32; ++x) acc[x] = 0.f;
+  for (int c = lane; c < cpr; c += 64) {
+    float hv[TW][8];
+#pragma unroll
+    for (int w = 0; w < TW; ++w)  // tokens past the last compute it again and store nothing
+      unpack8(*reinterpret_cast<const uint4*>(h + min(t0 + w, T - 1) * d + c * 8), hv[w]);
+#pragma unroll
+    for (int e = 0; e < EP; ++e) {  // experts past the last compute it again and are not picked
+      float gv[8];
+      unpack8(*reinterpret_cast<const uint4*>(gw + (int64_t)min(e, E - 1) * d + c * 8), gv);
+#pragma unroll
+      for (int w = 0; w < TW; ++w)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[w * EP + e] = add_rn(acc[w * EP + e], mul_rn(hv[w][i], gv[i]));
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < 16; ++x) acc[x] = halve<32>(acc[x], acc[x + 16]);
+#pragma unroll
+  for (int x = 0; x < 8; ++x) acc[x] = halve<16>(acc[x], acc[x + 8]);
+#pragma unroll
+  for (int x = 0; x < 4; ++x) acc[x] = halve<8>(acc[x], acc[x + 4]);
+#pragma unroll
+  for (int x = 0; x < 2; ++x) acc[x] = halve<4>(acc[x], acc[x + 2]);
+  const float logit = xor_sum<1>(halve<2>(acc[0], acc[1]));
+  const int64_t t = t0 + (lane >> 1) / EP;
+  const int e = (lane >> 1) % EP;
+  const bool valid = e < E;
+  // sigmoid score and biased logit of this lane's expert
+  const float score = valid ? 1.0f / (1.0f + expf(-logit)) : 0.f;
+  const float key = valid ? add_rn(logit, ebias[e]) : -INFINITY;
+  // top-k by repeated argmax over the token's lanes (ties: lowest expert index)
+  bool chosen = false;
+  int myk = -1;  // pick order of this lane's expert
+  float wsum = 0.f;
+  for (int k = 0; k < top_k; ++k) {
+    float best = chosen ? -INFINITY : key, bs = score;
+    int bi = valid && !chosen ? e : kMaxExperts;
+    auto step = [&](auto o) {
+      constexpr int O = decltype(o)::value;
+      const float ob = as_float(xor_partner<O>(__float_as_int(best)));
+      const float os = as_float(xor_partner<O>(__float_as_int(bs)));
+      const int oi = xor_partner<O>(bi);
+      if (ob > best || (ob == best && oi < bi)) {
+        best = ob;
+        bs = os;
+        bi = oi;
+      }
+    };
+    if constexpr (EP > 16) step(std::integral_constant<int, 32>{});
+    if constexpr (EP > 8) step(std::integral_constant<int, 16>{});
+    step(std::integral_constant<int, 8>{});
+    step(std::integral_constant<int, 4>{});
+    step(std::integral_constant<int, 2>{});
+    if (e == bi) { chosen = true; myk = k; }
+    wsum = add_rn(wsum, bi < kMaxExperts ? bs : 0.f);
+  }
+  float wgt = chosen ? score : 0.f;
+  if (top_k > 1) wgt = chosen ? wgt / add_rn(wsum, 1e-10f) : 0.f;
+  if (t >= T || (lane & 1)) return;
+  if (dense != nullptr) {
+    if (valid) dense[t * (E + S) + e] = wgt;
+    for (int s = e; s < S; s += EP) dense[t * (E + S) + E + s] = 1.0f;
+  }
+  if (topk_idx != nullptr && chosen) {
+    topk_idx[t * top_k + myk] = e;
+    topk_w[t * top_k + myk] = wgt;
+  }
+}
+
 // Small batches (decode): one workgroup of 4 waves per token, so that the
 // tokens spread over as many CUs as possible.
 // One token's gate: h_row (global or LDS) of d bf16 values; nthr threads
@@ -692,7 +802,16 @@ extern "C" int lfs_moe_route(const void* h, const void* gate_weight, const float
     hipLaunchKernelGGL(moe_route_token_kernel, dim3((unsigned)T), dim3(256), 0, (hipStream_t)stream,
                        (const uint16_t*)h, (const uint16_t*)gate_weight, expert_bias, down_bias, dense_weights,
                        bias_out, d, num_experts, num_shared, top_k, topk_idx, topk_weight);
-  else
+  else if (bias_out == nullptr && num_experts <= 32) {
+#define LFS_RR(EP)                                                                                                   \
+  hipLaunchKernelGGL(moe_route_rows_kernel<EP>, dim3((unsigned)((T + 128 / EP - 1) / (128 / EP))), dim3(256), 0,      \
+                     (hipStream_t)stream, (const uint16_t*)h, (const uint16_t*)gate_weight, expert_bias, dense_weights, \
+                     T, d, num_experts, num_shared, top_k, topk_idx, topk_weight)
+    if (num_experts <= 8) LFS_RR(8);
+    else if (num_experts <= 16) LFS_RR(16);
+    else LFS_RR(32);
+#undef LFS_RR
+  } else
     hipLaunchKernelGGL(moe_route_kernel, dim3((unsigned)((T + kRouteTokens - 1) / kRouteTokens)),
                        dim3(64 * kRouteTokens), 0, (hipStream_t)stream, (const uint16_t*)h,
                        (const uint16_t*)gate_weight, expert_bias, down_bias, dense_weights, bias_out, T, d,

@@ -103,15 +103,27 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_offsets_kernel(
   __shared__ int cnt[kAlignMaxExperts];
   __shared__ int off[kAlignMaxExperts + 1];
   const int tid = threadIdx.x, EE = E + S;
-  if (tid < EE) {
+  // one wave per expert scans its chunks' counts 64 at a time (one thread
+  // per expert waited a round trip per chunk: 11 us of a 16384-token dispatch)
+  const int lane = tid & 63;
+  for (int e = tid >> 6; e < EE; e += kAlignThreads / 64) {
     int run = 0;
-    for (int c = 0; c < chunks; ++c) {
-      const int v = hist[(int64_t)c * EE + tid];
-      hist[(int64_t)c * EE + tid] = run;
-      run += v;
+    for (int c0 = 0; c0 < chunks; c0 += 64) {
+      const int c = c0 + lane;
+      const int v = c < chunks ? hist[(int64_t)c * EE + e] : 0;
+      int incl = v;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += u;
+      }
+      if (c < chunks) hist[(int64_t)c * EE + e] = run + incl - v;
+      run += __shfl(incl, 63, 64);
     }
-    cnt[tid] = run;
-    cnt_out[tid] = run;
+    if (lane == 0) {
+      cnt[e] = run;
+      cnt_out[e] = run;
+    }
   }
   __syncthreads();
   if (tid == 0) {
@@ -167,57 +179,80 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_place_kernel(
   entry_row[i] = row;
 }
 
-// One workgroup per token, 8 consecutive columns per thread and pass.
-template <typename OutT>
+// 8 consecutive columns of one token per thread, the (token, column chunk)
+// pairs numbered through, so that every lane has work whatever d is (one
+// workgroup per token left 160 of 256 threads idle at d = 768 and held them
+// at a barrier for the token's entries).  The entries of a token are the same
+// addresses in all its lanes.  KK > 0: kk at compile time, so that all rows
+// and down biases are loaded before the first sum.
+template <typename OutT, int KK>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const OutT* __restrict__ out, int64_t ld,
                                                           const int32_t* __restrict__ entry_row,
                                                           const int64_t* __restrict__ topk_idx,
                                                           const float* __restrict__ topk_w, int top_k, int E,
                                                           int S, const float* __restrict__ b2, int d,
-                                                          uint16_t* __restrict__ y) {
-  const int t = blockIdx.x, kk = top_k + S;
-  __shared__ int rows[kAlignMaxExperts];
-  __shared__ int exs[kAlignMaxExperts];
-  __shared__ float wts[kAlignMaxExperts];
-  if ((int)threadIdx.x < kk) {
-    int tt, e;
-    float wt;
-    entry(topk_idx, topk_w, (int64_t)t * kk + threadIdx.x, kk, top_k, E, tt, e, wt);
-    rows[threadIdx.x] = entry_row[(int64_t)t * kk + threadIdx.x];
-    exs[threadIdx.x] = e;
-    wts[threadIdx.x] = wt;
-  }
-  __syncthreads();
-  for (int c = threadIdx.x * 8; c < d; c += 256 * 8) {
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int j = 0; j < kk; ++j) {
-      if (rows[j] < 0) continue;
-      float v[8];
-      if constexpr (sizeof(OutT) == 4) {
-        const float4* p = reinterpret_cast<const float4*>(out + (int64_t)rows[j] * ld + c);
-        const float4 a = p[0], b = p[1];
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-      } else {
-        unpack8(*reinterpret_cast<const uint4*>(out + (int64_t)rows[j] * ld + c), v);
-      }
+                                                          uint16_t* __restrict__ y, int64_t units) {
+  const int64_t u = blockIdx.x * 256ll + threadIdx.x;
+  if (u >= units) return;
+  const int cpr = d / 8, kk = KK > 0 ? KK : top_k + S;
+  const int64_t t = units >> 31 ? u / cpr : (int64_t)((unsigned)u / (unsigned)cpr);
+  const int c = (int)(u - t * cpr) * 8;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  auto add_row = [&](int row) {
+    float v[8];
+    if constexpr (sizeof(OutT) == 4) {
+      const float4* p = reinterpret_cast<const float4*>(out + (int64_t)row * ld + c);
+      const float4 a = p[0], b = p[1];
+      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    } else {
+      unpack8(*reinterpret_cast<const uint4*>(out + (int64_t)row * ld + c), v);
+    }
 #pragma unroll
-      for (int x = 0; x < 8; ++x) acc[x] += v[x];
+    for (int x = 0; x < 8; ++x) acc[x] += v[x];
+  };
+  auto add_bias = [&](int e, float wt) {
+    const float* bb = b2 + (int64_t)e * d + c;
+#pragma unroll
+    for (int x = 0; x < 8; ++x) acc[x] = fmaf(wt, bb[x], acc[x]);
+  };
+  if constexpr (KK > 0) {
+    int row[KK], ex[KK];
+    float wt[KK];
+#pragma unroll
+    for (int j = 0; j < KK; ++j) {
+      int tt;
+      entry(topk_idx, topk_w, t * KK + j, KK, top_k, E, tt, ex[j], wt[j]);
+      row[j] = entry_row[t * KK + j];
+    }
+#pragma unroll
+    for (int j = 0; j < KK; ++j)
+      if (row[j] >= 0) add_row(row[j]);
+    if (b2 != nullptr) {
+#pragma unroll
+      for (int j = 0; j < KK; ++j)
+        if (row[j] >= 0) add_bias(ex[j], wt[j]);
+    }
+  } else {
+    for (int j = 0; j < kk; ++j) {
+      const int row = entry_row[t * kk + j];
+      if (row >= 0) add_row(row);
     }
     if (b2 != nullptr) {
       for (int j = 0; j < kk; ++j) {
-        if (rows[j] < 0) continue;
-        const float* bb = b2 + (int64_t)exs[j] * d + c;
-#pragma unroll
-        for (int x = 0; x < 8; ++x) acc[x] = fmaf(wts[j], bb[x], acc[x]);
+        if (entry_row[t * kk + j] < 0) continue;
+        int tt, e;
+        float wt;
+        entry(topk_idx, topk_w, t * kk + j, kk, top_k, E, tt, e, wt);
+        add_bias(e, wt);
       }
     }
-    uint4 o;
-    o.x = pack_bf16x2(acc[0], acc[1]);
-    o.y = pack_bf16x2(acc[2], acc[3]);
-    o.z = pack_bf16x2(acc[4], acc[5]);
-    o.w = pack_bf16x2(acc[6], acc[7]);
-    *reinterpret_cast<uint4*>(y + (int64_t)t * d + c) = o;
   }
+  uint4 o;
+  o.x = pack_bf16x2(acc[0], acc[1]);
+  o.y = pack_bf16x2(acc[2], acc[3]);
+  o.z = pack_bf16x2(acc[4], acc[5]);
+  o.w = pack_bf16x2(acc[6], acc[7]);
+  *reinterpret_cast<uint4*>(y + t * d + c) = o;
 }
 
 // ------------------------------------------------ segment reduce (Triton) --
@@ -406,14 +441,25 @@ extern "C" int lfs_moe_combine(const void* out, int32_t out_is_f32, int64_t ld, 
   LFS_REQUIRE(out && entry_row && topk_idx && topk_weight && y, "moe_combine: null pointer");
   LFS_REQUIRE((((uintptr_t)out) | ((uintptr_t)y)) % 16 == 0, "moe_combine: buffers must be 16-byte aligned");
   LFS_REQUIRE(T < (1ll << 31), "moe_combine: too many tokens");
-  if (out_is_f32)
-    hipLaunchKernelGGL(moe_combine_kernel<float>, dim3((unsigned)T), dim3(256), 0, (hipStream_t)stream,
-                       (const float*)out, ld, entry_row, topk_idx, topk_weight, top_k, num_experts, num_shared,
-                       down_bias, d, (uint16_t*)y);
-  else
-    hipLaunchKernelGGL(moe_combine_kernel<uint16_t>, dim3((unsigned)T), dim3(256), 0, (hipStream_t)stream,
-                       (const uint16_t*)out, ld, entry_row, topk_idx, topk_weight, top_k, num_experts, num_shared,
-                       down_bias, d, (uint16_t*)y);
+  const int64_t units = T * (d / 8);
+#define LFS_MC(OT, KK)                                                                                              \
+  hipLaunchKernelGGL((moe_combine_kernel<OT, KK>), dim3((unsigned)((units + 255) / 256)), dim3(256), 0,              \
+                     (hipStream_t)stream, (const OT*)out, ld, entry_row, topk_idx, topk_weight, top_k, num_experts, \
+                     num_shared, down_bias, d, (uint16_t*)y, units)
+#define LFS_MCK(OT)                  \
+  switch (top_k + num_shared) {      \
+    case 2: LFS_MC(OT, 2); break;    \
+    case 3: LFS_MC(OT, 3); break;    \
+    case 5: LFS_MC(OT, 5); break;    \
+    default: LFS_MC(OT, 0); break;   \
+  }
+  if (out_is_f32) {
+    LFS_MCK(float)
+  } else {
+    LFS_MCK(uint16_t)
+  }
+#undef LFS_MCK
+#undef LFS_MC
   return check_launch("moe_combine");
 }
 

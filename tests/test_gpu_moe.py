@@ -209,3 +209,46 @@ def test_moe_route_large_batch_kernel_matches_per_token_kernel():
     # grouped-only call (no dense / bias outputs) gives the same picks
     _, _, idx, wt = K.moe_route(h, gw, eb, None, k, S, dense=False, return_topk=True)
     assert torch.equal(idx, big[2]) and torch.equal(wt, big[3])
+
+
+@pytest.mark.parametrize("E,S,k,d", [(1, 0, 1, 8), (5, 1, 2, 768), (8, 1, 2, 768), (8, 3, 8, 1032), (9, 0, 1, 512),
+                                     (16, 1, 2, 1024), (17, 2, 6, 520), (32, 1, 4, 768), (33, 1, 2, 768)])
+def test_moe_route_index_form_large_batch_same_bits(E, S, k, d):
+    """The gate without the routed bias above 1024 tokens (32 / 8, 16 or 32
+    tokens per wave) against the kernel of a workgroup per token on slices:
+    the same picks, weights and dense rows bit for bit, also on ties and at a
+    token count that leaves a wave part empty."""
+    T = 1029
+    g = torch.Generator(device=DEV).manual_seed(E * 100 + k)
+    h = torch.randn(T, d, generator=g, device=DEV).to(torch.bfloat16)
+    h[::50] = 0  # every logit 0: all ties
+    gate = (torch.randn(E, d, generator=g, device=DEV) / d ** 0.5).to(torch.bfloat16)
+    if E > 3:
+        gate[3] = gate[1]  # two experts with the same logits
+    bias = torch.randn(E, generator=g, device=DEV) * 0.01
+    bias[:min(E, 4)] = 0
+    res = K.moe_route(h, gate, bias, None, k, S, return_topk=True)
+    parts = [K.moe_route(h[i:i + 1000], gate, bias, None, k, S, return_topk=True) for i in (0, 1000)]
+    for got, want in zip((res[0], res[2], res[3]), zip(*[(p[0], p[2], p[3]) for p in parts])):
+        assert torch.equal(got, torch.cat(want))
+    only = K.moe_route(h, gate, bias, None, k, S, dense=False, return_topk=True)
+    assert torch.equal(only[2], res[2]) and torch.equal(only[3], res[3])
+
+
+@pytest.mark.parametrize("k,S,d", [(1, 0, 8), (2, 0, 264), (2, 1, 768), (4, 1, 768), (6, 2, 136)])
+def test_moe_combine_entry_counts(k, S, d):
+    """Every compiled entry count and the general loop, at column counts
+    that leave the last workgroup part empty, with dropped picks."""
+    rng = np.random.default_rng(k * 10 + S)
+    T, E = 37, 8
+    idx, w = picks(rng, T, E, k, bad=5)
+    rows = K.moe_align(dev(idx), dev(w), E, S)
+    _, _, _, er = MO.moe_align(idx, w, E, S)
+    b2 = rng.standard_normal((E + S, d)).astype(np.float32)
+    for dt in (torch.bfloat16, torch.float32):
+        out = dev(rng.standard_normal((rows.num_rows, d)).astype(np.float32)).to(dt)
+        for bias in (None, b2):
+            y = K.moe_combine(out, rows.entry_row, dev(idx), dev(w), E, S, None if bias is None else dev(bias))
+            ref = MO.moe_combine(out.double().cpu().numpy(), er, idx, w, E, S, np.zeros_like(b2) if bias is None else b2)
+            # one bf16 rounding of an fp32 sum vs of a float64 sum
+            assert np.all(np.abs(y.float().cpu().numpy() - ref) <= 2.0 ** -7 * np.abs(ref) + 1e-6)
