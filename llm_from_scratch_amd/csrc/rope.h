@@ -15,6 +15,13 @@ __device__ __forceinline__ float mul_rn(float a, float b) { return __fmul_rn(a, 
 __device__ __forceinline__ float add_rn(float a, float b) { return __fadd_rn(a, b); }
 __device__ __forceinline__ float sub_rn(float a, float b) { return __fsub_rn(a, b); }
 
+// One element pair of RoPE and its share of the sum of squares, with the
+// fused products spelled out: left to the compiler's contraction, which of
+// the two products is rounded on its own changes from kernel to kernel.
+__device__ __forceinline__ float rope_lo(float x1, float x2, float c, float s) { return fmaf(x1, c, -(x2 * s)); }
+__device__ __forceinline__ float rope_hi(float x1, float x2, float c, float s) { return fmaf(x1, s, x2 * c); }
+__device__ __forceinline__ float sum_sq(float a, float b) { return fmaf(a, a, b * b); }
+
 // Units per thread of qk_norm_rope_store.  A "unit" is one head's pair of
 // 8-element chunks (d0..d0+7 and D/2+d0..D/2+d0+7) that RoPE combines; q has
 // Hq*D/16 units, k Hkv*D/16.  Thread tid < 256 owns units tid, tid + 256,
@@ -128,7 +135,7 @@ struct RopeRow {
         unpack8(rb[i], b[i]);
         float s = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) s = add_rn(s, add_rn(mul_rn(a[i][e], a[i][e]), mul_rn(b[i][e], b[i][e])));
+        for (int e = 0; e < 8; ++e) s = add_rn(s, sum_sq(a[i][e], b[i][e]));
         if (isq) ssq = add_rn(ssq, s); else ssk = add_rn(ssk, s);
       }
     }
@@ -158,9 +165,8 @@ struct RopeRow {
           // norm output rounded to bf16 (the norm returns the input dtype)
           const float x1 = bf16_to_f32(f32_to_bf16(mul_rn(mul_rn(w1[i][e], a[i][e]), inv)));
           const float x2 = bf16_to_f32(f32_to_bf16(mul_rn(mul_rn(w2[i][e], b[i][e]), inv)));
-          const float c = c1[i][e], s = s1[i][e];
-          y1[e] = sub_rn(mul_rn(x1, c), mul_rn(x2, s));
-          y2[e] = add_rn(mul_rn(x2, c), mul_rn(x1, s));
+          y1[e] = rope_lo(x1, x2, c1[i][e], s1[i][e]);
+          y2[e] = rope_hi(x1, x2, c1[i][e], s1[i][e]);
         }
         uint4 o1, o2;
         o1.x = pack_bf16x2(y1[0], y1[1]); o1.y = pack_bf16x2(y1[2], y1[3]);

@@ -266,3 +266,25 @@ def test_moe_route_vs_reference_bf16_gate():
     assert not (differ & ~ties).any(), f"{int((differ & ~ties).sum())} tokens differ without a bf16 near-tie"
     assert differ.sum() <= 0.02 * len(differ)
     np.testing.assert_allclose(pw[~differ], ref_wts.float().numpy()[~differ], rtol=2 ** -6, atol=0)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(12, 4, 64), (16, 4, 64), (6, 2, 128), (5, 1, 16), (24, 8, 64), (32, 8, 128)])
+def test_qk_norm_rope_store_large_batch_same_bits(Hq, Hkv, D):
+    """One wave per token (512 tokens and up, at most 128 units a row) against
+    the workgroup-per-token form on slices of the same rows: strided rows,
+    positions outside the table, skipped and out-of-pool slots."""
+    T = 1030
+    g = torch.Generator(device=DEV).manual_seed(Hq * D)
+    qkv = torch.randn(T, (Hq + 2 * Hkv) * D + 8, generator=g, device=DEV).to(torch.bfloat16)[:, :(Hq + 2 * Hkv) * D]
+    qw, kw, cs = (torch.randn(n, generator=g, device=DEV) for n in (Hq * D, Hkv * D, 600 * D))
+    cs = cs.view(600, D)
+    pos = torch.randint(-3, 700, (T,), generator=g, device=DEV)
+    pool = (70, 16, Hkv, D)
+    slots = torch.randperm(70 * 16, generator=g, device=DEV)[:T].contiguous()
+    slots[::7], slots[5::90] = -1, 70 * 16
+    caches = [torch.full(pool, 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(4)]
+    q = K.qk_norm_rope_store(qkv, qw, kw, cs, pos, Hq, Hkv, 1e-5, caches[0], caches[1], slots)
+    want = torch.cat([K.qk_norm_rope_store(qkv[i:i + 500], qw, kw, cs, pos[i:i + 500], Hq, Hkv, 1e-5, caches[2],
+                                           caches[3], slots[i:i + 500]) for i in range(0, T, 500)])
+    assert torch.equal(q, want) and torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
+    assert torch.equal(K.qk_norm_rope_store(qkv, qw, kw, cs, pos, Hq, Hkv, 1e-5), want)
