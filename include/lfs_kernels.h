@@ -105,7 +105,7 @@
 extern "C" {
 #endif
 
-#define LFS_ABI_VERSION 15
+#define LFS_ABI_VERSION 16
 
 /* argument errors (negative); launch errors are positive hipError_t values */
 #define LFS_EINVAL (-1)
@@ -175,6 +175,15 @@ int lfs_fp8_gemm(const void* a, const float* a_s, const void* b, const float* b_
 int lfs_fp8_gemm_act_supported(int64_t M, int64_t N, int64_t K);
 int lfs_fp8_gemm_act(const void* a, int64_t lda, const void* b, const float* b_s, const float* bias,
                      int64_t bias_ld, void* c, int64_t M, int64_t N, int64_t K, void* stream);
+
+/*
+ * The same for at most 4 rows: c = lfs_fp8_gemm_skinny(act_quant(a, 128),
+ * b, b_s, bias) for bf16 a [M, K] with row stride lda (>= K, a multiple of
+ * 8), bit for bit, in one launch; every wave quantises its own K blocks.
+ * More rows are refused with LFS_EINVAL.
+ */
+int lfs_fp8_gemm_skinny_act(const void* a, int64_t lda, const void* b, const float* b_s, const float* bias,
+                            int64_t bias_ld, void* c, int64_t M, int64_t N, int64_t K, void* stream);
 
 /*
  * fp8_gemm with the K blocks split over `splits` workgroups per output tile

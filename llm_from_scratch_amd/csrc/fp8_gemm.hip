@@ -473,9 +473,22 @@ __global__ __launch_bounds__(BM * 2 * KS, KS == 1 ? 256 / BM : 1) void fp8_gemm_
 
 // KW waves of a group split the K blocks (4, or 8 / 16 for one 16-row tile
 // and long K: more K blocks in flight at once, still one launch).
-template <int MTW, int WGM, int KW = 4, int NT = 2>
+//
+// AQ: A is bf16 (rows lda elements apart) of at most kSkinnyActRows = 4 rows,
+// and every wave quantises its own K blocks: lane l takes 8 values of row
+// l / 16 (a 4 x 128 block is one 16-byte load per lane), and the codes go
+// through a wave-private LDS block into the operand layout.  The same
+// functions as act_quant and the same sums, so the result equals act_quant
+// then the form without AQ bit for bit.  It trades some 60 instructions and
+// two LDS trips per K block and wave for a launch: one row, K 2048, N 5632:
+// act_quant and GEMM back to back 6.96 -> 5.30 us (four rows 7.52 -> 5.32),
+// and half the host time of a linear called alone (26.6 -> 15.2 us).  More
+// rows would take another pass per K block in every workgroup.
+constexpr int kSkinnyActRows = 4;
+
+template <int MTW, int WGM, int KW = 4, int NT = 2, bool AQ = false>
 __global__ __launch_bounds__(64 * KW * WGM) void fp8_gemm_skinny(
-    const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ B,
+    const uint8_t* __restrict__ A, int64_t lda, const float* __restrict__ As, const uint8_t* __restrict__ B,
     const float* __restrict__ Bs, const float* __restrict__ bias, int64_t bias_ld, uint16_t* __restrict__ C,
     int M, int N, int K) {
   __shared__ __attribute__((aligned(16))) v4f red[WGM][KW][MTW][NT][64];
@@ -496,6 +509,10 @@ __global__ __launch_bounds__(64 * KW * WGM) void fp8_gemm_skinny(
     soff[mt] = m * (uint32_t)KT;
   }
   const float* bsrow = Bs + (size_t)(n0 / 128) * KT;  // the 16 NT columns share one 128-row scale block
+  static_assert(!AQ || (MTW == 1 && WGM == 1), "AQ: one 16-row tile");
+  __shared__ __attribute__((aligned(16))) uint8_t aq[AQ ? KW : 1][AQ ? kSkinnyActRows * BK : 1];
+  __shared__ float aqs[AQ ? KW : 1][kSkinnyActRows];
+  const uint16_t* xrow = reinterpret_cast<const uint16_t*>(A) + min(lane >> 4, M - 1) * lda + (lane & 15) * 8;
 
   v4f acc[MTW][NT];
 #pragma unroll
@@ -517,12 +534,34 @@ __global__ __launch_bounds__(64 * KW * WGM) void fp8_gemm_skinny(
     for (int nt = 0; nt < NT; ++nt) bf[nt] = ld(brow[nt] + (size_t)kb * BK);
 #pragma unroll
     for (int mt = 0; mt < MTW; ++mt) {
-      af[mt] = ld(A + aoff[mt] + (uint32_t)kb * BK);
-      sa[mt] = As[soff[mt] + kb];
+      if constexpr (AQ) {  // the raw values, in the buffer's first half
+        const u32x4 x = *reinterpret_cast<const u32x4*>(xrow + kb * BK);
+        af[mt] = __builtin_bit_cast(v8i, __builtin_shufflevector(x, x, 0, 1, 2, 3, 4, 5, 6, 7));
+      } else {
+        af[mt] = ld(A + aoff[mt] + (uint32_t)kb * BK);
+        sa[mt] = As[soff[mt] + kb];
+      }
     }
     sb = bsrow[kb];
   };
-  auto compute = [&](const v8i (&bf)[NT], const v8i (&af)[MTW], const float (&sa)[MTW], float sb) {
+  auto quantise = [&](v8i& a, float& sa) {  // AQ: raw values -> operand fragment and scale
+    uint4 x;
+    x.x = a[0], x.y = a[1], x.z = a[2], x.w = a[3];
+    float f[8], amax = 0.f;
+    unpack8(x, f);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(f[i]));
+    const float s = scale_from_amax(group_max<16>(amax), false);
+    wave_lds_fence();  // the block before has been read
+    *reinterpret_cast<uint2*>(&aq[kw][lane * 8]) = quant8(f, s);
+    if ((lane & 15) == 0) aqs[kw][lane >> 4] = s;
+    wave_lds_fence();
+    const int row = r16 % kSkinnyActRows;  // rows past M repeat row M - 1 and are not stored
+    a = ld(&aq[kw][row * BK + g * 16]);
+    sa = aqs[kw][row];
+  };
+  auto compute = [&](const v8i (&bf)[NT], v8i (&af)[MTW], float (&sa)[MTW], float sb) {
+    if constexpr (AQ) quantise(af[0], sa[0]);
 #pragma unroll
     for (int mt = 0; mt < MTW; ++mt) {
       const float sc = sa[mt] * sb;
@@ -1712,6 +1751,41 @@ extern "C" int lfs_fp8_grouped_gemm(const void* a, const float* a_s, int64_t a_r
   return check_launch("fp8_grouped_gemm");
 }
 
+namespace {
+template <bool AQ>
+void launch_skinny(const void* a, int64_t lda, const float* a_s, const void* b, const float* b_s, const float* bias,
+                   int64_t bias_ld, void* c, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+  const int mt = (int)((M + 15) / 16);
+  const int KT = (int)(K / 128);
+  // N <= 4096 (<= 128 groups of 32 columns): groups of 16 columns, twice
+  // the workgroups, each re-reading all M activation rows.  Measured back to
+  // back: M = 16, K 1024 / N 4096 4.8 -> 3.9 us, K 4096 / N 1024 9.5 -> 7.3
+  // us; M = 128, K 768 / N 1280 7.9 -> 6.7 us, K 1024 / N 4096 10.8 -> 9.6
+  // us; but M = 16, N = 5632 (176 groups of 32) 6.6 -> 7.4 us
+  const bool narrow = N <= 4096;
+  const dim3 grid((unsigned)((N + (narrow ? 15 : 31)) / (narrow ? 16 : 32)));
+#define LFS_SK(MTW, WGM, KW, NT)                                                                                \
+  hipLaunchKernelGGL((fp8_gemm_skinny<MTW, WGM, KW, NT, AQ>), grid, dim3(64 * KW * WGM), 0, st,                 \
+                     (const uint8_t*)a, lda, a_s, (const uint8_t*)b, b_s, bias, bias_ld, (uint16_t*)c, (int)M,   \
+                     (int)N, (int)K)
+  // one 16-row tile: the K blocks over 16 / 8 / 4 waves (>= 1.5 blocks per wave)
+  if (narrow && mt <= 1 && KT >= 24) LFS_SK(1, 1, 16, 1);
+  else if (narrow && mt <= 1 && KT >= 12) LFS_SK(1, 1, 8, 1);
+  else if (narrow && mt <= 1) LFS_SK(1, 1, 4, 1);
+  else if (mt <= 1 && KT >= 24) LFS_SK(1, 1, 16, 2);
+  else if (mt <= 1 && KT >= 12) LFS_SK(1, 1, 8, 2);
+  else if (mt <= 1) LFS_SK(1, 1, 4, 2);
+  else if constexpr (AQ) return;  // (not reached: at most kSkinnyActRows rows)
+  else if (narrow && mt <= 2) LFS_SK(2, 1, 4, 1);
+  else if (narrow && mt <= 4) LFS_SK(4, 1, 4, 1);
+  else if (narrow) LFS_SK(4, 2, 4, 1);
+  else if (mt <= 2) LFS_SK(2, 1, 4, 2);
+  else if (mt <= 4) LFS_SK(4, 1, 4, 2);
+  else LFS_SK(4, 2, 4, 2);
+#undef LFS_SK
+}
+}  // namespace
+
 extern "C" int lfs_fp8_gemm_skinny(const void* a, const float* a_s, const void* b, const float* b_s,
                                    const float* bias, int64_t bias_ld, void* c, int64_t M, int64_t N, int64_t K,
                                    void* stream) {
@@ -1723,33 +1797,23 @@ extern "C" int lfs_fp8_gemm_skinny(const void* a, const float* a_s, const void* 
   LFS_REQUIRE(K > 0 && a && a_s && b && b_s && c, "fp8_gemm_skinny: null pointer");
   LFS_REQUIRE((((uintptr_t)a | (uintptr_t)b) & 15u) == 0, "fp8_gemm_skinny: a and b must be 16-byte aligned");
   LFS_REQUIRE(bias_ld == 0 || (bias != nullptr && bias_ld >= N), "fp8_gemm_skinny: bias_ld must be 0 or >= N");
-  hipStream_t st = (hipStream_t)stream;
-  const int mt = (int)((M + 15) / 16);
-  const int KT = (int)(K / 128);
-  // N <= 4096 (<= 128 groups of 32 columns): groups of 16 columns, twice
-  // the workgroups, each re-reading all M activation rows.  Measured back to
-  // back: M = 16, K 1024 / N 4096 4.8 -> 3.9 us, K 4096 / N 1024 9.5 -> 7.3
-  // us; M = 128, K 768 / N 1280 7.9 -> 6.7 us, K 1024 / N 4096 10.8 -> 9.6
-  // us; but M = 16, N = 5632 (176 groups of 32) 6.6 -> 7.4 us
-  const bool narrow = N <= 4096;
-  const dim3 grid((unsigned)((N + (narrow ? 15 : 31)) / (narrow ? 16 : 32)));
-#define LFS_SK(MTW, WGM, KW, NT)                                                                                \
-  hipLaunchKernelGGL((fp8_gemm_skinny<MTW, WGM, KW, NT>), grid, dim3(64 * KW * WGM), 0, st, (const uint8_t*)a,   \
-                     a_s, (const uint8_t*)b, b_s, bias, bias_ld, (uint16_t*)c, (int)M, (int)N, (int)K)
-  // one 16-row tile: the K blocks over 16 / 8 / 4 waves (>= 1.5 blocks per wave)
-  if (narrow && mt <= 1 && KT >= 24) LFS_SK(1, 1, 16, 1);
-  else if (narrow && mt <= 1 && KT >= 12) LFS_SK(1, 1, 8, 1);
-  else if (narrow && mt <= 1) LFS_SK(1, 1, 4, 1);
-  else if (mt <= 1 && KT >= 24) LFS_SK(1, 1, 16, 2);
-  else if (mt <= 1 && KT >= 12) LFS_SK(1, 1, 8, 2);
-  else if (mt <= 1) LFS_SK(1, 1, 4, 2);
-  else if (narrow && mt <= 2) LFS_SK(2, 1, 4, 1);
-  else if (narrow && mt <= 4) LFS_SK(4, 1, 4, 1);
-  else if (narrow) LFS_SK(4, 2, 4, 1);
-  else if (mt <= 2) LFS_SK(2, 1, 4, 2);
-  else if (mt <= 4) LFS_SK(4, 1, 4, 2);
-  else LFS_SK(4, 2, 4, 2);
-#undef LFS_SK
+  launch_skinny<false>(a, K, a_s, b, b_s, bias, bias_ld, c, M, N, K, (hipStream_t)stream);
   return check_launch("fp8_gemm_skinny");
+}
+
+extern "C" int lfs_fp8_gemm_skinny_act(const void* a, int64_t lda, const void* b, const float* b_s, const float* bias,
+                                       int64_t bias_ld, void* c, int64_t M, int64_t N, int64_t K, void* stream) {
+  LFS_REQUIRE(M >= 0 && N >= 0 && K >= 0, "fp8_gemm_skinny_act: negative shape");
+  LFS_REQUIRE(M <= kSkinnyActRows, "fp8_gemm_skinny_act: M=%lld must be <= %d", (long long)M, kSkinnyActRows);
+  LFS_REQUIRE(K % 128 == 0, "fp8_gemm_skinny_act: K=%lld must be a multiple of 128", (long long)K);
+  LFS_REQUIRE(N < (1ll << 31) && K < (1ll << 24), "fp8_gemm_skinny_act: shape too large");
+  if (M == 0 || N == 0) return 0;
+  LFS_REQUIRE(K > 0 && a && b && b_s && c, "fp8_gemm_skinny_act: null pointer");
+  LFS_REQUIRE(lda >= K && lda % 8 == 0,
+              "fp8_gemm_skinny_act: the row stride lda=%lld must be >= K and a multiple of 8", (long long)lda);
+  LFS_REQUIRE((((uintptr_t)a | (uintptr_t)b) & 15u) == 0, "fp8_gemm_skinny_act: a and b must be 16-byte aligned");
+  LFS_REQUIRE(bias_ld == 0 || (bias != nullptr && bias_ld >= N), "fp8_gemm_skinny_act: bias_ld must be 0 or >= N");
+  launch_skinny<true>(a, lda, nullptr, b, b_s, bias, bias_ld, c, M, N, K, (hipStream_t)stream);
+  return check_launch("fp8_gemm_skinny_act");
 }
 

@@ -59,7 +59,12 @@ class FP8Linear(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x = x.to(torch.bfloat16).contiguous()
-        if self.fused_act(x.numel() // self.in_features):
+        rows = x.numel() // self.in_features
+        if (0 < rows <= kernels.SKINNY_ACT_MAX_M and x.data_ptr() % 16 == 0
+                and kernels.use_skinny_gemm(rows, self.out_features, self.in_features)):
+            # a few rows: act_quant inside the skinny GEMM's waves, the same bits
+            return kernels.fp8_gemm_skinny_act(x, self.weight, self.weight_scale, self.bias)
+        if self.fused_act(rows):
             # act_quant inside the GEMM's workgroups: the same codes, scales and bits
             return kernels.fp8_gemm_act(x, self.weight, self.weight_scale, self.bias)
         xq, xs = kernels.act_quant(x, 128)

@@ -291,6 +291,36 @@ def fp8_gemm_act(x: torch.Tensor, b: torch.Tensor, b_s: torch.Tensor,
     return c
 
 
+SKINNY_ACT_MAX_M = 4  # rows that fp8_gemm_skinny_act quantises inside the GEMM
+
+
+def fp8_gemm_skinny_act(x: torch.Tensor, b: torch.Tensor, b_s: torch.Tensor,
+                        bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """fp8_gemm(*act_quant(x, 128), b, b_s, bias) for at most
+    SKINNY_ACT_MAX_M rows in one launch, bit for bit: every wave quantises
+    the K blocks it multiplies.  x: bf16 [..., K] (rows may be strided, K
+    contiguous)."""
+    assert x.stride(-1) == 1, "x must be contiguous along K"
+    _on_gpu(x, b, b_s)
+    _dtype(x, torch.bfloat16, "x")
+    _dtype(b, FP8, "b")
+    _dtype(b_s, torch.float32, "b_s")
+    K = x.size(-1)
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
+    M, N = x2.size(0), b.size(0)
+    assert b.dim() == 2 and b.size(1) == K and b.is_contiguous(), "b must be contiguous [N, K]"
+    assert b_s.shape == (math.ceil(N / 128), K // 128) and b_s.is_contiguous(), "b_s must be [ceil(N/128), K/128]"
+    if bias is not None:
+        _on_gpu(x, bias)
+        _dtype(bias, torch.float32, "bias")
+        assert bias.is_contiguous() and bias.shape == (N,), "bias must be fp32 [N]"
+    c = x.new_empty(*x.shape[:-1], N, dtype=torch.bfloat16)
+    rc = _lib.load().lfs_fp8_gemm_skinny_act(_ptr(x2), x2.stride(0) if M > 1 else K, _ptr(b), _ptr(b_s), _ptr(bias), 0,
+                                             _ptr(c), M, N, K, _stream(x))
+    _lib.check(rc, "fp8_gemm_skinny_act")
+    return c
+
+
 # ------------------------------------------------------------- paged KV path --
 def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
                   v_cache: torch.Tensor, slot_mapping: torch.Tensor) -> None:

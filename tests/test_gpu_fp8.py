@@ -12,6 +12,7 @@ import torch
 
 from llm_from_scratch_amd import kernels as K
 from llm_from_scratch_amd import workloads as W
+from llm_from_scratch_amd.fp8_linear import FP8Linear
 from oracle import fp8 as F
 
 pytestmark = pytest.mark.gpu
@@ -347,6 +348,38 @@ def test_fp8_gemm_act_equals_act_quant_then_gemm(M, N, Kd, variant):
         torch.cuda.synchronize()
         assert torch.equal(got.view(torch.int16), ref.view(torch.int16)), f"{M}x{N}x{Kd} bias={bb is not None}"
         assert_close(f32(got), gemm_oracle(xq, xs, b, b_s, bb), f"fp8_gemm_act {M}x{N}x{Kd}")
+
+
+@pytest.mark.parametrize("N,Kd", [(16, 128), (1344, 512), (1000, 1536), (4096, 3072), (5632, 2048), (4100, 1408),
+                                  (6001, 3200)])
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+def test_fp8_gemm_skinny_act_bit_identical(M, N, Kd):
+    """act_quant inside the skinny GEMM's waves (every K split and column
+    width) against act_quant then fp8_gemm: strided rows, outliers, an
+    all-zero group, with and without bias; FP8Linear takes it."""
+    x = torch.randn(M, Kd + 24, generator=torch.Generator(device=DEV).manual_seed(M * N), device=DEV)
+    x[:, ::37] *= 40
+    x[-1, :128] = 0
+    x = x.to(torch.bfloat16)[:, :Kd]
+    w = (torch.randn(N, Kd, generator=torch.Generator(device=DEV).manual_seed(N), device=DEV) * 0.02).to(torch.bfloat16)
+    wq, ws = K.weight_quant(w)
+    bias = torch.randn(N, generator=torch.Generator(device=DEV).manual_seed(Kd), device=DEV)
+    xq, xs = K.act_quant(x.contiguous())
+    for bv in (None, bias):
+        assert torch.equal(K.fp8_gemm_skinny_act(x, wq, ws, bv), K.fp8_gemm(xq, xs, wq, ws, bv))
+    lin = FP8Linear(Kd, N, bias=True, device=DEV)
+    lin.load_weight(w, bias)
+    assert torch.equal(lin(x.reshape(1, M, Kd)), K.fp8_gemm(xq, xs, wq, ws, bias).view(1, M, N))
+
+
+def test_fp8_gemm_skinny_act_rejects_other_shapes():
+    b, b_s = torch.zeros(256, 256, device=DEV, dtype=torch.float8_e4m3fn), torch.ones(2, 2, device=DEV)
+    with pytest.raises(ValueError, match="must be <= 4"):
+        K.fp8_gemm_skinny_act(torch.zeros(5, 256, device=DEV, dtype=torch.bfloat16), b, b_s)
+    with pytest.raises(ValueError, match="row stride"):
+        K.fp8_gemm_skinny_act(torch.zeros(3, 260, device=DEV, dtype=torch.bfloat16)[:, :256], b, b_s)
+    with pytest.raises(ValueError, match="aligned"):
+        K.fp8_gemm_skinny_act(torch.zeros(1, 264, device=DEV, dtype=torch.bfloat16)[:, 2:258], b, b_s)
 
 
 def test_fp8_gemm_act_rejects_other_shapes():
