@@ -58,7 +58,9 @@ class FP8Linear(nn.Module):
         return kernels.weight_dequant(self.weight, self.weight_scale, 128)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        x = x.to(torch.bfloat16).contiguous()
+        if x.dtype != torch.bfloat16:
+            x = x.to(torch.bfloat16)
+        x = x.contiguous()
         rows = x.numel() // self.in_features
         if (0 < rows <= kernels.SKINNY_ACT_MAX_M and x.data_ptr() % 16 == 0
                 and kernels.use_skinny_gemm(rows, self.out_features, self.in_features)):
