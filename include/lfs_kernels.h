@@ -436,6 +436,17 @@ int lfs_qk_norm_rope_store(const void* qkv, int64_t ld, const float* q_weight, c
                            int64_t num_slots, int64_t max_positions, float eps, void* stream);
 
 /*
+ * The same, and with k_out and v_out (bf16 [T, Hkv, D], both or neither) the
+ * rotated k and the v rows in token order as well, for an attention over
+ * whole prompts whose keys would otherwise be gathered back from the slots.
+ */
+int lfs_qk_norm_rope_store_kv(const void* qkv, int64_t ld, const float* q_weight, const float* k_weight,
+                              const float* cos_sin, const int64_t* positions, const int64_t* slot_mapping,
+                              void* q_out, void* k_cache, void* v_cache, void* k_out, void* v_out, int64_t T,
+                              int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t num_slots,
+                              int64_t max_positions, float eps, void* stream);
+
+/*
  * moe_route, per token t of h: bf16 [T, d]:
  *   logit[e] = h[t] . gate_weight[e] (fp32), gate_weight bf16 [E, d];
  *   the top_k experts by logit + expert_bias[e] (ties: lower index) get

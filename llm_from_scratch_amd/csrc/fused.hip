@@ -221,8 +221,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(
     const uint16_t* __restrict__ qkv, int64_t ld, const float* __restrict__ qw,
     const float* __restrict__ kw, const float* __restrict__ cos_sin, const int64_t* __restrict__ pos,
     const int64_t* __restrict__ slots, uint16_t* __restrict__ q_out, uint16_t* __restrict__ kc,
-    uint16_t* __restrict__ vc, int Hq, int Hkv, int D, int64_t num_slots, int64_t max_pos,
-    float eps) {
+    uint16_t* __restrict__ vc, uint16_t* __restrict__ k_out, uint16_t* __restrict__ v_out, int Hq, int Hkv, int D,
+    int64_t num_slots, int64_t max_pos, float eps) {
   __shared__ float red[8];
   const int64_t t = blockIdx.x;
   const uint16_t* row = qkv + t * ld;
@@ -232,27 +232,27 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(
   const float* cs = cos_sin + p * D;  // [cos(0..D/2) | sin(0..D/2)]
   const int64_t slot = slots != nullptr ? slots[t] : -1;
   const bool store = slot >= 0 && slot < num_slots;
-  // v: straight copy into the cache slot (Hkv*D/8 chunks)
-  if (store) {
-    const int64_t dst = slot * (int64_t)Hkv * D;
-    for (int c = threadIdx.x; c < Hkv * D / 8; c += 256)
-      *reinterpret_cast<uint4*>(vc + dst + c * 8) =
-          *reinterpret_cast<const uint4*>(row + (Hq + Hkv) * D + c * 8);
+  // v: straight copy into the cache slot (Hkv*D/8 chunks), and to v_out
+  for (int c = threadIdx.x; c < Hkv * D / 8; c += 256) {
+    const uint4 x = *reinterpret_cast<const uint4*>(row + (Hq + Hkv) * D + c * 8);
+    if (store) *reinterpret_cast<uint4*>(vc + slot * (int64_t)Hkv * D + c * 8) = x;
+    if (v_out != nullptr) *reinterpret_cast<uint4*>(v_out + t * Hkv * D + c * 8) = x;
   }
   RopeRow<kRopeUPT> rr;
   rr.load(row, Hq, Hkv, D, threadIdx.x);
   rr.load_weights(qw, kw);
   rr.load_rope(cs);
   rr.finish(eps, red, [&](bool isq, int h, int d0, const uint4& o1, const uint4& o2) {
-    uint16_t* dst;
+    auto put = [&](uint16_t* dst) {
+      *reinterpret_cast<uint4*>(dst + d0) = o1;
+      *reinterpret_cast<uint4*>(dst + half + d0) = o2;
+    };
     if (isq) {
-      dst = q_out + (t * Hq + h) * D;
+      put(q_out + (t * Hq + h) * D);
     } else {
-      if (!store) return;
-      dst = kc + (slot * Hkv + h) * D;
+      if (store) put(kc + (slot * Hkv + h) * D);
+      if (k_out != nullptr) put(k_out + (t * Hkv + h) * D);
     }
-    *reinterpret_cast<uint4*>(dst + d0) = o1;
-    *reinterpret_cast<uint4*>(dst + half + d0) = o2;
   });
 }
 
@@ -266,8 +266,8 @@ template <int NU>
 __global__ __launch_bounds__(256) void qk_norm_rope_store_rows_kernel(
     const uint16_t* __restrict__ qkv, int64_t ld, const float* __restrict__ qw, const float* __restrict__ kw,
     const float* __restrict__ cos_sin, const int64_t* __restrict__ pos, const int64_t* __restrict__ slots,
-    uint16_t* __restrict__ q_out, uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, int64_t T, int Hq, int Hkv,
-    int D, int64_t num_slots, int64_t max_pos, float eps) {
+    uint16_t* __restrict__ q_out, uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, uint16_t* __restrict__ k_out,
+    uint16_t* __restrict__ v_out, int64_t T, int Hq, int Hkv, int D, int64_t num_slots, int64_t max_pos, float eps) {
   const int lane = threadIdx.x & 63, half = D / 2, upr = D / 16, uq = Hq * upr, un = (Hq + Hkv) * upr;
   // the unit's place in a row: q then k, element d0 of head h
   bool isq[NU];
@@ -301,10 +301,11 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_rows_kernel(
       load8(cs + d0[i], c1[i]);
       load8(cs + half + d0[i], s1[i]);
     }
-    if (store)  // v: straight copy into the cache slot
-      for (int c = lane; c < Hkv * D / 8; c += 64)
-        *reinterpret_cast<uint4*>(vc + slot * (int64_t)Hkv * D + c * 8) =
-            *reinterpret_cast<const uint4*>(row + (Hq + Hkv) * D + c * 8);
+    for (int c = lane; c < Hkv * D / 8; c += 64) {  // v: straight copy into the cache slot, and to v_out
+      const uint4 x = *reinterpret_cast<const uint4*>(row + (Hq + Hkv) * D + c * 8);
+      if (store) *reinterpret_cast<uint4*>(vc + slot * (int64_t)Hkv * D + c * 8) = x;
+      if (v_out != nullptr) *reinterpret_cast<uint4*>(v_out + t * Hkv * D + c * 8) = x;
+    }
     float tq = 0.f, tk = 0.f;
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_rows_kernel(
     const float invk = rsqrtf(add_rn(mul_rn(tk, 1.0f / (float)(Hkv * D)), eps));
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
-      if (lane + 64 * i >= un || (!isq[i] && !store)) continue;
+      if (lane + 64 * i >= un) continue;
       const float inv = isq[i] ? invq : invk;
       float y1[8], y2[8];
 #pragma unroll
@@ -329,11 +330,20 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_rows_kernel(
         y1[e] = rope_lo(x1, x2, c1[i][e], s1[i][e]);
         y2[e] = rope_hi(x1, x2, c1[i][e], s1[i][e]);
       }
-      uint16_t* dst = (isq[i] ? q_out + (t * Hq + h[i]) * D : kc + (slot * Hkv + h[i]) * D) + d0[i];
-      *reinterpret_cast<uint4*>(dst) = make_uint4(pack_bf16x2(y1[0], y1[1]), pack_bf16x2(y1[2], y1[3]),
-                                                  pack_bf16x2(y1[4], y1[5]), pack_bf16x2(y1[6], y1[7]));
-      *reinterpret_cast<uint4*>(dst + half) = make_uint4(pack_bf16x2(y2[0], y2[1]), pack_bf16x2(y2[2], y2[3]),
-                                                         pack_bf16x2(y2[4], y2[5]), pack_bf16x2(y2[6], y2[7]));
+      const uint4 o1 = make_uint4(pack_bf16x2(y1[0], y1[1]), pack_bf16x2(y1[2], y1[3]), pack_bf16x2(y1[4], y1[5]),
+                                  pack_bf16x2(y1[6], y1[7]));
+      const uint4 o2 = make_uint4(pack_bf16x2(y2[0], y2[1]), pack_bf16x2(y2[2], y2[3]), pack_bf16x2(y2[4], y2[5]),
+                                  pack_bf16x2(y2[6], y2[7]));
+      auto put = [&](uint16_t* dst) {
+        *reinterpret_cast<uint4*>(dst + d0[i]) = o1;
+        *reinterpret_cast<uint4*>(dst + half + d0[i]) = o2;
+      };
+      if (isq[i]) {
+        put(q_out + (t * Hq + h[i]) * D);
+      } else {
+        if (store) put(kc + (slot * Hkv + h[i]) * D);
+        if (k_out != nullptr) put(k_out + (t * Hkv + h[i]) * D);
+      }
     }
   }
 }
@@ -846,6 +856,17 @@ extern "C" int lfs_qk_norm_rope_store(const void* qkv, int64_t ld, const float* 
                                       int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                                       int64_t num_slots, int64_t max_positions, float eps,
                                       void* stream) {
+  return lfs_qk_norm_rope_store_kv(qkv, ld, q_weight, k_weight, cos_sin, positions, slot_mapping, q_out, k_cache,
+                                   v_cache, nullptr, nullptr, T, num_q_heads, num_kv_heads, head_dim, num_slots,
+                                   max_positions, eps, stream);
+}
+
+extern "C" int lfs_qk_norm_rope_store_kv(const void* qkv, int64_t ld, const float* q_weight, const float* k_weight,
+                                         const float* cos_sin, const int64_t* positions,
+                                         const int64_t* slot_mapping, void* q_out, void* k_cache, void* v_cache,
+                                         void* k_out, void* v_out, int64_t T, int32_t num_q_heads,
+                                         int32_t num_kv_heads, int32_t head_dim, int64_t num_slots,
+                                         int64_t max_positions, float eps, void* stream) {
   const int Hq = num_q_heads, Hkv = num_kv_heads, D = head_dim;
   LFS_REQUIRE(T >= 0 && Hq > 0 && Hkv > 0, "qk_norm_rope_store: bad shape");
   LFS_REQUIRE(D % 16 == 0 && D > 0 && D <= 512, "qk_norm_rope_store: head_dim=%d must be a multiple of 16", D);
@@ -857,7 +878,9 @@ extern "C" int lfs_qk_norm_rope_store(const void* qkv, int64_t ld, const float* 
   LFS_REQUIRE(qkv && q_weight && k_weight && cos_sin && positions && q_out,
               "qk_norm_rope_store: null pointer");
   LFS_REQUIRE(slot_mapping == nullptr || (k_cache && v_cache), "qk_norm_rope_store: null cache");
-  LFS_REQUIRE(((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0,
+  LFS_REQUIRE((k_out == nullptr) == (v_out == nullptr), "qk_norm_rope_store: k_out and v_out go together");
+  LFS_REQUIRE(((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)k_out |
+               (uintptr_t)v_out) % 16 == 0,
               "qk_norm_rope_store: buffers must be 16-byte aligned");
   const int units = (Hq + Hkv) * (D / 16);
   if (T >= kRopeRowsT && units <= 128) {
@@ -865,7 +888,8 @@ extern "C" int lfs_qk_norm_rope_store(const void* qkv, int64_t ld, const float* 
 #define LFS_QR(NU)                                                                                                  \
   hipLaunchKernelGGL(qk_norm_rope_store_rows_kernel<NU>, grid, dim3(256), 0, (hipStream_t)stream,                    \
                      (const uint16_t*)qkv, ld, q_weight, k_weight, cos_sin, positions, slot_mapping, (uint16_t*)q_out, \
-                     (uint16_t*)k_cache, (uint16_t*)v_cache, T, Hq, Hkv, D, num_slots, max_positions, eps)
+                     (uint16_t*)k_cache, (uint16_t*)v_cache, (uint16_t*)k_out, (uint16_t*)v_out, T, Hq, Hkv, D, num_slots,          \
+                     max_positions, eps)
     if (units <= 64) LFS_QR(1);
     else LFS_QR(2);
 #undef LFS_QR
@@ -873,8 +897,8 @@ extern "C" int lfs_qk_norm_rope_store(const void* qkv, int64_t ld, const float* 
   }
   hipLaunchKernelGGL(qk_norm_rope_store_kernel, dim3((unsigned)T), dim3(256), 0, (hipStream_t)stream,
                      (const uint16_t*)qkv, ld, q_weight, k_weight, cos_sin, positions, slot_mapping,
-                     (uint16_t*)q_out, (uint16_t*)k_cache, (uint16_t*)v_cache, Hq, Hkv, D, num_slots,
-                     max_positions, eps);
+                     (uint16_t*)q_out, (uint16_t*)k_cache, (uint16_t*)v_cache, (uint16_t*)k_out, (uint16_t*)v_out, Hq, Hkv,
+                     D, num_slots, max_positions, eps);
   return check_launch("qk_norm_rope_store");
 }
 

@@ -200,18 +200,17 @@ class PagedGQAAttention(nn.Module):
             if trace is not None:
                 trace.update(qkv=qkv, q=q, att_o=o, att_out=out)
             return out
+        whole = ctx.is_prefill and ctx.block_tables is None  # whole prompts: the keys of this very call
         q = kernels.qk_norm_rope_store(qkv, self.q_norm.weight, self.k_norm.weight, self.rope.cos_sin_cached,
                                        positions, self.num_heads, self.num_kv_heads, self.q_norm.eps,
-                                       self.k_cache, self.v_cache, ctx.slot_mapping)
+                                       self.k_cache, self.v_cache, ctx.slot_mapping, return_kv=whole)
         if ctx.is_prefill:
             if ctx.block_tables is not None:  # prefix-cache hit: keys from the pool
                 o = kernels.flash_attn_varlen_func(q, self.k_cache, self.v_cache, ctx.cu_seqlens_q,
                                                    ctx.cu_seqlens_k, ctx.max_seqlen_q, ctx.max_seqlen_k,
                                                    self.scale, block_table=ctx.block_tables)
-            else:  # whole prompts: the keys just stored, in slot order
-                flat = (-1, self.num_kv_heads, self.head_dim)
-                k = self.k_cache.view(flat)[ctx.slot_mapping]
-                v = self.v_cache.view(flat)[ctx.slot_mapping]
+            else:
+                q, k, v = q
                 o = kernels.flash_attn_varlen_func(q, k, v, ctx.cu_seqlens_q, ctx.cu_seqlens_k,
                                                    ctx.max_seqlen_q, ctx.max_seqlen_k, self.scale)
             o = o.reshape(T, -1)

@@ -845,14 +845,16 @@ def qk_norm_rope_store(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight: torc
                        cos_sin: torch.Tensor, positions: torch.Tensor, num_q_heads: int,
                        num_kv_heads: int, eps: float, k_cache: Optional[torch.Tensor] = None,
                        v_cache: Optional[torch.Tensor] = None,
-                       slot_mapping: Optional[torch.Tensor] = None) -> torch.Tensor:
+                       slot_mapping: Optional[torch.Tensor] = None, return_kv: bool = False):
     """q_norm / k_norm (fp32 RMSNorm over Hq*D and Hkv*D), half-split RoPE
     (model/attention/utils.py:34-45) and the KV slot write, one launch.
 
     qkv: bf16 [T, (Hq + 2 Hkv) * D] (rows may be strided); cos_sin: fp32
     [max_pos, D] = cat(cos, sin); positions int64 [T]; caches bf16
     [NB, BS, Hkv, D] and slot_mapping int64 [T] (-1 = skip), or None.
-    Returns q: bf16 [T, Hq, D].
+    Returns q: bf16 [T, Hq, D]; with ``return_kv`` (q, k, v), the rotated k
+    and the v rows bf16 [T, Hkv, D] as written to the slots (an attention
+    over whole prompts then need not gather them back from the pool).
     """
     assert qkv.dim() == 2 and qkv.stride(1) == 1
     T = qkv.size(0)
@@ -876,12 +878,14 @@ def qk_norm_rope_store(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight: torc
         assert slot_mapping.numel() == T and slot_mapping.is_contiguous()
         num_slots = k_cache.shape[0] * k_cache.shape[1]
     q = torch.empty(T, num_q_heads, D, dtype=torch.bfloat16, device=qkv.device)
-    rc = _lib.load().lfs_qk_norm_rope_store(
+    k = torch.empty(T, num_kv_heads, D, dtype=torch.bfloat16, device=qkv.device) if return_kv else None
+    v = torch.empty_like(k) if return_kv else None
+    rc = _lib.load().lfs_qk_norm_rope_store_kv(
         _ptr(qkv), qkv.stride(0), _ptr(q_weight), _ptr(k_weight), _ptr(cos_sin), _ptr(positions),
-        _ptr(slot_mapping), _ptr(q), _ptr(k_cache), _ptr(v_cache), T, num_q_heads, num_kv_heads, D,
+        _ptr(slot_mapping), _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(k), _ptr(v), T, num_q_heads, num_kv_heads, D,
         num_slots, cos_sin.size(0), float(eps), _stream(qkv))
     _lib.check(rc, "qk_norm_rope_store")
-    return q
+    return (q, k, v) if return_kv else q
 
 
 def moe_route(h: torch.Tensor, gate_weight: torch.Tensor, expert_bias: torch.Tensor,

@@ -288,3 +288,12 @@ def test_qk_norm_rope_store_large_batch_same_bits(Hq, Hkv, D):
                                            caches[3], slots[i:i + 500]) for i in range(0, T, 500)])
     assert torch.equal(q, want) and torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
     assert torch.equal(K.qk_norm_rope_store(qkv, qw, kw, cs, pos, Hq, Hkv, 1e-5), want)
+    # k and v in token order: what the slots hold, and every token's where slots are skipped
+    stored = (slots >= 0) & (slots < 70 * 16)
+    for n in (T, 300):  # both forms
+        q3, k3, v3 = K.qk_norm_rope_store(qkv[:n], qw, kw, cs, pos[:n], Hq, Hkv, 1e-5, caches[2], caches[3], slots[:n],
+                                          return_kv=True)
+        assert torch.equal(q3, want[:n]) and torch.equal(v3.view(n, -1), qkv[:n, (Hq + Hkv) * D:])
+        at = slots[:n][stored[:n]]
+        assert torch.equal(k3[stored[:n]], caches[0].view(-1, Hkv, D)[at])
+        assert torch.equal(k3, K.qk_norm_rope_store(qkv[:n], qw, kw, cs, pos[:n], Hq, Hkv, 1e-5, return_kv=True)[1])
