@@ -201,6 +201,22 @@ __device__ __forceinline__ float xor_max(float v) {
   }
 }
 
+// One halving of two sums: lanes with bit O of the lane id clear get
+// a + a(lane ^ O), the others b + b(lane ^ O) -- what xor_sum<O> gives them
+// for a or for b, in one exchange for both.
+template <int O>
+__device__ __forceinline__ float halve(float a, float b) {  // lane & O ? b(lane ^ O) + b : a + a(lane ^ O)
+  if constexpr (O == 32 || O == 16) {
+    const auto r = O == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_int(a), __float_as_int(b), false, false)
+                           : __builtin_amdgcn_permlane16_swap(__float_as_int(a), __float_as_int(b), false, false);
+    return as_float((int)r[0]) + as_float((int)r[1]);
+  } else {
+    const bool up = __lane_id() & O;
+    const float give = up ? a : b, keep = up ? b : a;
+    return keep + as_float(xor_partner<O>(__float_as_int(give)));
+  }
+}
+
 // xor-butterfly over groups of W consecutive lanes (W a power of two <= 64),
 // distances W/2 down to 1 (the order of the sums)
 template <int W>

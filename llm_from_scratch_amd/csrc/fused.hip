@@ -500,19 +500,6 @@ __global__ __launch_bounds__(64 * kRouteTokens) void moe_route_kernel(
 // picks its token's top k.  16384 tokens, d 768, 8 experts: 39 -> 13 us
 // against a wave per token, which waits out its loads, its eight butterflies
 // and its picks one after the other.
-template <int O>
-__device__ __forceinline__ float halve(float a, float b) {  // lane & O ? b(lane ^ O) + b : a + a(lane ^ O)
-  if constexpr (O == 32 || O == 16) {
-    const auto r = O == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_int(a), __float_as_int(b), false, false)
-                           : __builtin_amdgcn_permlane16_swap(__float_as_int(a), __float_as_int(b), false, false);
-    return as_float((int)r[0]) + as_float((int)r[1]);
-  } else {
-    const bool up = __lane_id() & O;
-    const float give = up ? a : b, keep = up ? b : a;
-    return keep + as_float(xor_partner<O>(__float_as_int(give)));
-  }
-}
-
 template <int EP>
 __global__ __launch_bounds__(256) void moe_route_rows_kernel(const uint16_t* __restrict__ h,
                                                              const uint16_t* __restrict__ gw,

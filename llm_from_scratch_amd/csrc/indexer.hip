@@ -7,12 +7,20 @@
 // d <= 128, zero-padded to 128), fp32 everywhere after.  A 16-head block of
 // q[b, m] is the first operand and a 16-key block of k[b] the second, so
 // lane l ends with key (l % 16) and heads 4(l / 16) .. +3 of the block: the
-// ReLU, the head weights and three of the head sums stay in the lane, the
-// rest is two xor shuffles (16, 32).
+// ReLU, the head weights and three of the head sums stay in the lane; the
+// sums of four key blocks then meet by halving (lane distance 16, 32), which
+// leaves lane l with key l of the 64, a whole line per store.
 //
-// One workgroup per (b, 8 queries, chunk of IDX_NCHUNK keys), one wave per
+// Bound: the VALU beside the MFMAs.  A score costs a multiply that clamps to
+// [0, 1] (ReLU: |q . k| < 2^25, so the scores are taken times 2^-25, exactly)
+// and an fma; the scale comes back as 2^12 in the weights and 2^13 at the end,
+// powers of two, so the same bits for every weight between 2^-95 and 2^115.
+// fmaxf cost two v_max_f32 (the first quiets a signaling NaN), which run at
+// half the rate of a multiply: 1 x 4096 x 4096, 64 heads, D 128: 190 -> 173 us.
+//
+// One workgroup per (b, 8 queries, chunk of nchunk keys), one wave per
 // query; the wave keeps its query's H/16 operand fragments in registers.
-// The chunk's keys pass through LDS in tiles of 64, loaded once for the
+// The chunk's keys pass through LDS in tiles of 128, loaded once for the
 // eight waves (double-buffered, the next tile's global loads in flight
 // during the current tile's MFMAs).  Operand K bytes: lane l supplies
 // 16-byte chunks g and g + 4 (g = l / 16) of the 128-byte row for both q
@@ -26,9 +34,17 @@ namespace {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr int IDX_NCHUNK = 512;  // keys per workgroup
-constexpr int IDX_QPW = 8;       // queries (waves) per workgroup
-constexpr int IDX_KT = 64;       // keys per LDS tile
+constexpr int IDX_QPW = 8;  // queries (waves) per workgroup
+// Keys per LDS tile: a barrier each, and the next tile's loads have one tile
+// of MFMAs to land (4096 x 4096, 64 heads: 64 keys 151 us, 128 144, 256 143).
+constexpr int IDX_KT = 128;
+// Keys per workgroup, a multiple of the tile: every workgroup loads its
+// queries first (64 KB at 64 heads of 128), so as many as still leave four
+// workgroups per CU, two rounds (4096 x 4096: 512 keys 173 us, 1024 158, 2048
+// 151, 4096 the same); below that short chunks, to spread a few queries'
+// keys over the CUs.
+constexpr int IDX_CHUNKS[] = {2048, 1024, 512, 256};
+constexpr int64_t IDX_MIN_WG = 1024;
 
 // byte offset of 16-byte chunk c of key row r in an LDS tile of D-byte rows
 template <int D>
@@ -42,7 +58,7 @@ template <int HB, int D>  // HB: 16-head blocks
 __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
     const uint8_t* __restrict__ q, const float* __restrict__ q_s, const uint8_t* __restrict__ k,
     const float* __restrict__ k_s, float* __restrict__ o, int M, int N, int H, int64_t k_stride_b,
-    int64_t ks_stride_b) {
+    int64_t ks_stride_b, int nchunk) {
   constexpr int CPR = D / 16;                 // 16-byte chunks per key row
   constexpr int TCH = IDX_KT * CPR;           // chunks per LDS tile
   constexpr int NT = 64 * IDX_QPW;
@@ -51,8 +67,8 @@ __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int b = blockIdx.z, m = blockIdx.y * IDX_QPW + wave;
   const bool active = m < M;  // inactive waves still take part in the barriers
-  const int n_begin = blockIdx.x * IDX_NCHUNK;
-  const int n_end = min(N, n_begin + IDX_NCHUNK);
+  const int n_begin = blockIdx.x * nchunk;
+  const int n_end = min(N - n_begin, nchunk) + n_begin;
   const int c16 = lane & 15, g = lane >> 4;
   const bool lo_ok = 16 * g < D, hi_ok = 16 * (g + 4) < D;  // this lane's chunks g, g + 4 exist
 
@@ -74,7 +90,7 @@ __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int hr = hb * 16 + 4 * g + r;
-      qw[hb][r] = hr < H ? q_s[qrow + hr] : 0.f;
+      qw[hb][r] = hr < H ? q_s[qrow + hr] * 0x1p12f : 0.f;
     }
   }
 
@@ -111,25 +127,30 @@ __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
     if (active) {
       const uint8_t* tile = kt[buf];
 #pragma unroll
-      for (int st = 0; st < IDX_KT / 16; ++st) {
-        const int r = 16 * st + c16;
-        uint4 lo = make_uint4(0, 0, 0, 0), hi = make_uint4(0, 0, 0, 0);
-        if (lo_ok) lo = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g));
-        if (hi_ok) hi = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g + 4));
-        const v8i kf = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-        float acc = 0.f;
+      for (int k64 = 0; k64 < IDX_KT; k64 += 64) {
+        float sum[4];
 #pragma unroll
-        for (int hb = 0; hb < HB; ++hb) {
-          const v4f z = {0.f, 0.f, 0.f, 0.f};
-          // D[head][key]: lane holds key c16, heads hb*16 + 4g .. +3
-          const v4f s = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qf[hb], kf, z, 0, 0, 0, 0, 0, 0);
+        for (int st = 0; st < 4; ++st) {
+          const int r = k64 + 16 * st + c16;
+          uint4 lo = make_uint4(0, 0, 0, 0), hi = make_uint4(0, 0, 0, 0);
+          if (lo_ok) lo = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g));
+          if (hi_ok) hi = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g + 4));
+          const v8i kf = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+          float acc = 0.f;
 #pragma unroll
-          for (int x = 0; x < 4; ++x) acc = fmaf(fmaxf(s[x], 0.f), qw[hb][x], acc);
+          for (int hb = 0; hb < HB; ++hb) {
+            const v4f z = {0.f, 0.f, 0.f, 0.f};
+            // D[head][key]: lane holds key c16, heads hb*16 + 4g .. +3
+            const v4f s = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qf[hb], kf, z, 0, 0, 0, 0, 0, 0);
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+              acc = fmaf(__builtin_amdgcn_fmed3f(s[x] * 0x1p-25f, 0.f, 1.f), qw[hb][x], acc);
+          }
+          sum[st] = acc;
         }
-        acc += __shfl_xor(acc, 16, 64);
-        acc += __shfl_xor(acc, 32, 64);
-        const int n = t0 + 16 * st + c16;
-        if (g == 0 && n < n_end) orow[n] = acc * ksb[n];
+        const float tot = halve<32>(halve<16>(sum[0], sum[1]), halve<16>(sum[2], sum[3]));
+        const int n = t0 + k64 + lane;
+        if (n < n_end) orow[n] = (tot * 0x1p13f) * ksb[n];
       }
     }
     if (ti + 1 < ntiles) store_tile(kr, buf ^ 1);  // buffer buf ^ 1 was last read in tile ti - 1
@@ -154,14 +175,20 @@ extern "C" int lfs_fp8_index(const void* q, const float* q_s, const void* k, con
   LFS_REQUIRE(((((uintptr_t)q) | ((uintptr_t)k)) & 15u) == 0 && (k_stride_b % 16) == 0,
               "fp8_index: q and k rows must be 16-byte aligned");
   LFS_REQUIRE(B < 65536 && (M + IDX_QPW - 1) / IDX_QPW < 65536, "fp8_index: grid too large");
-  const dim3 grid((unsigned)((N + IDX_NCHUNK - 1) / IDX_NCHUNK), (unsigned)((M + IDX_QPW - 1) / IDX_QPW),
-                  (unsigned)B);
+  const int64_t rows = B * ((M + IDX_QPW - 1) / IDX_QPW);
+  int nchunk = IDX_KT;
+  for (const int c : IDX_CHUNKS)
+    if (rows * (((int64_t)N + c - 1) / c) >= IDX_MIN_WG) {
+      nchunk = c;
+      break;
+    }
+  const dim3 grid((unsigned)(((int64_t)N + nchunk - 1) / nchunk), (unsigned)((M + IDX_QPW - 1) / IDX_QPW), (unsigned)B);
   hipStream_t st = (hipStream_t)stream;
   const int hb = (H + 15) / 16;
   const uint8_t *qq = (const uint8_t*)q, *kk = (const uint8_t*)k;
 #define LFS_IX(HB, DD)                                                                                       \
   hipLaunchKernelGGL((fp8_index_kernel<HB, DD>), grid, dim3(64 * IDX_QPW), 0, st, qq, q_s, kk, k_s, o, M, N, H, \
-                     k_stride_b, ks_stride_b)
+                     k_stride_b, ks_stride_b, nchunk)
 #define LFS_IXD(HB)                    \
   case HB:                             \
     if (D == 128) LFS_IX(HB, 128);     \

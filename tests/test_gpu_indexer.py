@@ -77,3 +77,43 @@ def test_fp8_index_reference_pipeline():
     full = np.maximum(np.einsum("bmhd,bnd->bmhn", qf, kf), 0) * (w * D ** -0.5).cpu().numpy()
     approx = full.sum(2)
     assert np.abs(o - approx).max() < 0.1 * np.abs(approx).max()
+
+
+@pytest.mark.parametrize("B,M,N,H,D", [
+    (1, 1, 129, 16, 128),     # one query: chunks of one tile
+    (1, 2048, 1025, 16, 64),  # chunks of 256, the last of one key
+    (2, 1024, 1500, 16, 32),  # 512
+    (1, 4096, 2049, 32, 64),  # 1024
+    (1, 8200, 130, 16, 128),  # 2048: one chunk, a part tile and a part workgroup of queries
+])
+def test_fp8_index_chunk_lengths(B, M, N, H, D):
+    """Every key chunk length the sizes choose, at part tiles and chunks, with
+    small and large head weights of both signs: a score depends on its own
+    query and key alone, so the same bits as calls of a few queries over
+    slices of the keys (one-tile chunks, which the tests above hold against
+    the oracle)."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    q, k = ((torch.randn(*s, generator=g, device=DEV) * 100).clamp(-448, 448).to(torch.float8_e4m3fn)
+            for s in ((B, M, H, D), (B, N, D)))
+    for scale in (1.0, 2.0 ** -60, 2.0 ** 60):
+        qs = (torch.rand(B, M, H, generator=g, device=DEV) - 0.2) * scale
+        ks = torch.rand(B, N, generator=g, device=DEV)
+        o = K.fp8_index(q, qs, k, ks)
+        for m in (0, max(0, M // 2 - 3), max(0, M - 11)):
+            for n in (0, max(0, N - 140)):
+                part = K.fp8_index(q[:, m:m + 11].contiguous(), qs[:, m:m + 11], k[:, n:n + 140], ks[:, n:n + 140])
+                assert torch.equal(o[:, m:m + 11, n:n + 140], part), (scale, m, n)
+        assert torch.isfinite(o).all()
+
+
+def test_fp8_index_nan_codes_score_zero():
+    """A NaN code makes its products NaN, which the ReLU takes as 0."""
+    g = torch.Generator(device=DEV).manual_seed(1)
+    q, k = (torch.randn(*s, generator=g, device=DEV).to(torch.float8_e4m3fn) for s in ((1, 9, 32, 64), (1, 200, 64)))
+    qs, ks = torch.rand(1, 9, 32, generator=g, device=DEV), torch.rand(1, 200, generator=g, device=DEV)
+    want = K.fp8_index(q, qs, k, ks)
+    k.view(torch.uint8)[0, 77, 5] = 0x7F
+    k.view(torch.uint8)[0, 150, 60] = 0xFF
+    o = K.fp8_index(q, qs, k, ks)
+    want[0, :, [77, 150]] = 0
+    assert torch.equal(o, want)
