@@ -180,6 +180,37 @@ def test_swiglu_quant(T, E, F):
     torch.testing.assert_close(qs, want_s, rtol=2e-7, atol=0)
 
 
+@pytest.mark.parametrize("T,E,F", [(8200, 1, 512), (2049, 1, 128), (1031, 2, 384), (683, 3, 640)])
+def test_swiglu_quant_large_batch_same_bits(T, E, F):
+    """The (row, chunk) form of large batches against the wave-per-row form on
+    slices: part workgroups, gates beyond the fast range, NaN and infinities."""
+    g = torch.Generator(device=DEV).manual_seed(T)
+    h13 = (torch.randn(T, E, 2, F, generator=g, device=DEV) * 4).to(torch.bfloat16)
+    h13[::5, :, 0, ::9] *= 30
+    for i, x in enumerate((float("nan"), float("inf"), -float("inf"), -0.0, 60.0, -60.25)):
+        h13[7 * i + 1, 0, 0, 3::40] = x
+    route = torch.rand(T, E, generator=g, device=DEV)
+    q, qs = K.swiglu_quant(h13, route)
+    parts = [K.swiglu_quant(h13[i:i + 600].contiguous(), route[i:i + 600]) for i in range(0, T, 600)]
+    assert torch.equal(q.view(torch.uint8), torch.cat([p[0] for p in parts]).view(torch.uint8))
+    assert torch.equal(qs.view(torch.int32), torch.cat([p[1] for p in parts]).view(torch.int32))
+
+
+@pytest.mark.parametrize("up", [1.0, -2.0 ** 100])
+def test_swiglu_quant_every_gate_value_same_bits(up):
+    """A row per bf16 gate value, whose scale then holds silu's bits (the up
+    factor lifts the smallest above the scale's floor) and whose codes hold its
+    sign: the large-batch form against the wave-per-row form."""
+    pat = torch.arange(65536, device=DEV).to(torch.int16).view(torch.bfloat16)
+    h13 = torch.stack([pat.view(-1, 1).expand(-1, 128), torch.full((65536, 128), up, device=DEV, dtype=torch.bfloat16)],
+                      1).view(65536, 1, 2, 128).contiguous()
+    route = torch.ones(65536, 1, device=DEV)
+    q, qs = K.swiglu_quant(h13, route)
+    parts = [K.swiglu_quant(h13[i:i + 2000], route[i:i + 2000]) for i in range(0, 65536, 2000)]
+    assert torch.equal(q.view(torch.uint8), torch.cat([p[0] for p in parts]).view(torch.uint8))
+    assert torch.equal(qs.view(torch.int32), torch.cat([p[1] for p in parts]).view(torch.int32))
+
+
 @pytest.mark.parametrize("T,d,E,S,top_k,with_res", [(128, 768, 8, 1, 2, True), (37, 1024, 16, 2, 4, False),
                                                     (9, 2048, 8, 0, 1, True), (5, 4096, 32, 1, 3, True),
                                                     (64, 512, 4, 0, 1, True), (3, 1024, 6, 2, 2, False)])
