@@ -14,9 +14,13 @@
 // Bound: the VALU beside the MFMAs.  A score costs a multiply that clamps to
 // [0, 1] (ReLU: |q . k| < 2^25, so the scores are taken times 2^-25, exactly)
 // and an fma; the scale comes back as 2^12 in the weights and 2^13 at the end,
-// powers of two, so the same bits for every weight between 2^-95 and 2^115.
-// fmaxf cost two v_max_f32 (the first quiets a signaling NaN), which run at
-// half the rate of a multiply: 1 x 4096 x 4096, 64 heads, D 128: 190 -> 173 us.
+// powers of two.  fmaxf costs two v_max_f32 (the first quiets a signaling
+// NaN), which run at half the rate of a multiply: 1 x 4096 x 4096, 64 heads,
+// D 128: 190 -> 173 us.  The same bits as fmaxf while no weight makes a
+// product lose bits below 2^-149 or a sum pass 2^128 on one scale and not on
+// the other: every weight 0 or in [2^-95, 2^95) (scores are multiples of
+// 2^-18, at most 128 of them meet).  A query with any other weight -- larger,
+// smaller, infinite, NaN -- takes fmaxf and its weights unscaled.
 //
 // One workgroup per (b, 8 queries, chunk of nchunk keys), one wave per
 // query; the wave keeps its query's H/16 operand fragments in registers.
@@ -26,6 +30,8 @@
 // 16-byte chunks g and g + 4 (g = l / 16) of the 128-byte row for both q
 // and k -- the same permutation of the head dim on both sides -- so the
 // sixteen rows of one LDS read hit every bank once with the swizzle below.
+#include <type_traits>
+
 #include "common.h"
 
 namespace lfs {
@@ -45,6 +51,12 @@ constexpr int IDX_KT = 128;
 // keys over the CUs.
 constexpr int IDX_CHUNKS[] = {2048, 1024, 512, 256};
 constexpr int64_t IDX_MIN_WG = 1024;
+
+// head weights whose scores may be summed on the scale of 2^-13 (see above)
+__device__ __forceinline__ bool weight_scales(float w) {
+  const unsigned e = (__float_as_uint(w) >> 23) & 0xFF;
+  return (e >= 127 - 95 && e < 127 + 95) || w == 0.f;
+}
 
 // byte offset of 16-byte chunk c of key row r in an LDS tile of D-byte rows
 template <int D>
@@ -76,6 +88,7 @@ __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
   // the heads this lane's results belong to
   v8i qf[HB];
   float qw[HB][4];
+  bool scaled = true;
   const int64_t qrow = ((int64_t)b * M + min(m, M - 1)) * H;
 #pragma unroll
   for (int hb = 0; hb < HB; ++hb) {
@@ -90,9 +103,15 @@ __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int hr = hb * 16 + 4 * g + r;
-      qw[hb][r] = hr < H ? q_s[qrow + hr] * 0x1p12f : 0.f;
+      qw[hb][r] = hr < H ? q_s[qrow + hr] : 0.f;
+      scaled = scaled && weight_scales(qw[hb][r]);
     }
   }
+  scaled = __all(scaled);  // the wave's lanes hold all heads of its query
+#pragma unroll
+  for (int hb = 0; hb < HB; ++hb)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) qw[hb][r] *= scaled ? 0x1p12f : 1.f;
 
   const uint8_t* kb = k + (int64_t)b * k_stride_b;
   const float* ksb = k_s + (int64_t)b * ks_stride_b;
@@ -115,6 +134,38 @@ __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
     }
   };
 
+  // the wave's scores against the tile in buffer buf, whose first key is t0
+  auto scores = [&](auto scale, int t0, int buf) {
+    constexpr bool SC = decltype(scale)::value;
+    const uint8_t* tile = kt[buf];
+#pragma unroll
+    for (int k64 = 0; k64 < IDX_KT; k64 += 64) {
+      float sum[4];
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        const int r = k64 + 16 * st + c16;
+        uint4 lo = make_uint4(0, 0, 0, 0), hi = make_uint4(0, 0, 0, 0);
+        if (lo_ok) lo = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g));
+        if (hi_ok) hi = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g + 4));
+        const v8i kf = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+        float acc = 0.f;
+#pragma unroll
+        for (int hb = 0; hb < HB; ++hb) {
+          const v4f z = {0.f, 0.f, 0.f, 0.f};
+          // D[head][key]: lane holds key c16, heads hb*16 + 4g .. +3
+          const v4f s = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qf[hb], kf, z, 0, 0, 0, 0, 0, 0);
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+            acc = fmaf(SC ? __builtin_amdgcn_fmed3f(s[x] * 0x1p-25f, 0.f, 1.f) : fmaxf(s[x], 0.f), qw[hb][x], acc);
+        }
+        sum[st] = acc;
+      }
+      const float tot = halve<32>(halve<16>(sum[0], sum[1]), halve<16>(sum[2], sum[3]));
+      const int n = t0 + k64 + lane;
+      if (n < n_end) orow[n] = (SC ? tot * 0x1p13f : tot) * ksb[n];
+    }
+  };
+
   const int ntiles = (n_end - n_begin + IDX_KT - 1) / IDX_KT;
   uint4 kr[CPT];
   load_tile(kr, n_begin);
@@ -125,33 +176,8 @@ __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
     const int buf = ti & 1;
     if (ti + 1 < ntiles) load_tile(kr, t0 + IDX_KT);
     if (active) {
-      const uint8_t* tile = kt[buf];
-#pragma unroll
-      for (int k64 = 0; k64 < IDX_KT; k64 += 64) {
-        float sum[4];
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          const int r = k64 + 16 * st + c16;
-          uint4 lo = make_uint4(0, 0, 0, 0), hi = make_uint4(0, 0, 0, 0);
-          if (lo_ok) lo = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g));
-          if (hi_ok) hi = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g + 4));
-          const v8i kf = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-          float acc = 0.f;
-#pragma unroll
-          for (int hb = 0; hb < HB; ++hb) {
-            const v4f z = {0.f, 0.f, 0.f, 0.f};
-            // D[head][key]: lane holds key c16, heads hb*16 + 4g .. +3
-            const v4f s = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qf[hb], kf, z, 0, 0, 0, 0, 0, 0);
-#pragma unroll
-            for (int x = 0; x < 4; ++x)
-              acc = fmaf(__builtin_amdgcn_fmed3f(s[x] * 0x1p-25f, 0.f, 1.f), qw[hb][x], acc);
-          }
-          sum[st] = acc;
-        }
-        const float tot = halve<32>(halve<16>(sum[0], sum[1]), halve<16>(sum[2], sum[3]));
-        const int n = t0 + k64 + lane;
-        if (n < n_end) orow[n] = (tot * 0x1p13f) * ksb[n];
-      }
+      if (scaled) scores(std::true_type{}, t0, buf);
+      else scores(std::false_type{}, t0, buf);
     }
     if (ti + 1 < ntiles) store_tile(kr, buf ^ 1);  // buffer buf ^ 1 was last read in tile ti - 1
     __syncthreads();

@@ -117,3 +117,25 @@ def test_fp8_index_nan_codes_score_zero():
     o = K.fp8_index(q, qs, k, ks)
     want[0, :, [77, 150]] = 0
     assert torch.equal(o, want)
+
+
+@pytest.mark.parametrize("e", [-140, -126, -110, -96, -95, 0, 94, 95, 110, 116])
+def test_fp8_index_any_head_weight(e):
+    """Weights over the whole fp32 range: one head of weight w and score s
+    gives fp32(s * w) (the other heads add exact zeros: weight 0, or a score
+    that the ReLU sets to 0 whatever its weight)."""
+    rng = np.random.default_rng(e + 200)
+    B, M, N, H, D = 1, 11, 150, 20, 64
+    qi = rng.choice(np.arange(-4, 5, dtype=np.float32), (B, M, H, D))
+    qi[:, :, 0] = -1  # only negative products
+    ki = rng.choice(np.arange(1, 5, dtype=np.float32), (B, N, D))
+    qi[:, :, 7, 0] = 4
+    w = np.float32(np.ldexp(1 + 2.0 ** -23, e))
+    qs = np.zeros((B, M, H), np.float32)
+    qs[:, :, 7] = w
+    qs[:, 1, 7] *= -1
+    qs[:, ::2, 0] = np.float32(2.0 ** 120)  # a negative score under a huge weight
+    qs[:, 3, 0] = np.float32(2.0 ** -130)
+    o = K.fp8_index(codes(qi), torch.from_numpy(qs).to(DEV), codes(ki), torch.ones(B, N, device=DEV))
+    s = np.maximum(np.einsum("bmd,bnd->bmn", qi[:, :, 7].astype(np.float64), ki), 0)
+    np.testing.assert_array_equal(o.cpu().numpy(), (s * qs[:, :, 7, None].astype(np.float64)).astype(np.float32))
