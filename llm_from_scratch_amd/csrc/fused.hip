@@ -549,6 +549,10 @@ __global__ __launch_bounds__(256) void moe_route_rows_kernel(const uint16_t* __r
   bool chosen = false;
   int myk = -1;  // pick order of this lane's expert
   float wsum = 0.f;
+  // A NaN key beats and loses to nothing, so the lanes may end with different
+  // picks; the sum then takes the score that expert 0's lane picked, as the
+  // kernel of a whole wave per token does.
+  const bool odd = __any(key != key);
   for (int k = 0; k < top_k; ++k) {
     float best = chosen ? -INFINITY : key, bs = score;
     int bi = valid && !chosen ? e : kMaxExperts;
@@ -569,7 +573,13 @@ __global__ __launch_bounds__(256) void moe_route_rows_kernel(const uint16_t* __r
     step(std::integral_constant<int, 4>{});
     step(std::integral_constant<int, 2>{});
     if (e == bi) { chosen = true; myk = k; }
-    wsum = add_rn(wsum, bi < kMaxExperts ? bs : 0.f);
+    if (odd) {
+      const int base = lane & -(2 * EP), lead = __shfl(bi, base, 64);
+      bs = __shfl(score, base + 2 * (lead < kMaxExperts ? lead : 0), 64);
+      wsum = add_rn(wsum, bs * (bi < kMaxExperts ? 1.f : 0.f));
+    } else {
+      wsum = add_rn(wsum, bi < kMaxExperts ? bs : 0.f);
+    }
   }
   float wgt = chosen ? score : 0.f;
   if (top_k > 1) wgt = chosen ? wgt / add_rn(wsum, 1e-10f) : 0.f;

@@ -235,6 +235,28 @@ def test_moe_route_index_form_large_batch_same_bits(E, S, k, d):
     assert torch.equal(only[2], res[2]) and torch.equal(only[3], res[3])
 
 
+@pytest.mark.parametrize("E,k", [(8, 2), (16, 4), (32, 4)])
+def test_moe_route_nan_gate_same_weights(E, k):
+    """NaN in a gate row or in the selection bias (one expert, the first or
+    another): the form without the routed bias gives the weights of the form
+    with it, bit for bit, above 1024 tokens."""
+    T, S, d = 2050, 1, 256
+    g = torch.Generator(device=DEV).manual_seed(E)
+    h = torch.randn(T, d, generator=g, device=DEV).to(torch.bfloat16)
+    gate = torch.randn(E, d, generator=g, device=DEV).to(torch.bfloat16)
+    bias, b2 = (torch.randn(*n, generator=g, device=DEV) for n in ((E,), (E + S, d)))
+    for e, in_bias in ((0, False), (3, False), (2, True), (None, True)):
+        gw, eb = gate.clone(), bias.clone()
+        if in_bias:
+            eb[2 if e is None else e] = float("nan") if e is not None else float("inf")
+        else:
+            gw[e, 5] = float("nan")
+        want = K.moe_route(h, gw, eb, b2, k, S)[0]
+        got = K.moe_route(h, gw, eb, None, k, S)[0]
+        nan = want.isnan()
+        assert torch.equal(nan, got.isnan()) and torch.equal(want[~nan], got[~nan]), (e, in_bias)
+
+
 @pytest.mark.parametrize("k,S,d", [(1, 0, 8), (2, 0, 264), (2, 1, 768), (4, 1, 768), (6, 2, 136)])
 def test_moe_combine_entry_counts(k, S, d):
     """Every compiled entry count and the general loop, at column counts
