@@ -66,6 +66,11 @@ typedef __attribute__((address_space(3))) uint8_t lds_u8;
 constexpr int KT = 64;               // keys per tile
 constexpr int NW = 4;                // waves per workgroup
 constexpr int RW = 32;               // rows (query token, head) per wave
+// Workgroups per grid row: a launch takes less than 2^32 threads in x (a few
+// prompts padded to a long max_seqlen_q pass that: 2^24 workgroups).  A
+// multiple of 8, so the id in x fixes the XCD.  Ids past the last work item
+// fall past the last tile.
+constexpr int64_t kGridX = 1 << 20;
 
 // N copies of 16 bytes per lane, from base + off[c] (per lane) to LDS address
 // lds + 1024 c + 16 * lane.  The kernel waits for them before its barrier
@@ -207,7 +212,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
   // 8 XCDs: XCD x takes kv head x / xsplit (xsplit = 8 / Hkv where Hkv divides
   // 8: every xsplit-th row tile of it), so that a pair's K and V are read
   // through one or few L2s and ragged sequences still load the XCDs evenly.
-  int rank = blockIdx.x, kh;
+  int rank = blockIdx.y * gridDim.x + blockIdx.x, kh;
   if (xsplit > 0) {
     kh = (rank & 7) / xsplit;
     rank = (rank >> 3) * xsplit + ((rank & 7) - kh * xsplit);
@@ -477,8 +482,9 @@ extern "C" int lfs_prefill_attention(const void* q, const void* k, const void* v
   const int64_t rtiles = ((int64_t)max_seqlen_q * G + RW * NW - 1) / (RW * NW);
   const int xsplit = Hkv <= 8 && 8 % Hkv == 0 ? 8 / Hkv : 0;
   const int64_t nt = xsplit > 0 ? (rtiles + xsplit - 1) / xsplit * xsplit : rtiles;
-  LFS_REQUIRE(B * nt < (1ll << 31) / Hkv && Hkv < 65536, "prefill_attention: grid too large");
-  const dim3 grid((unsigned)(B * nt * Hkv));
+  LFS_REQUIRE(B * nt < ((1ll << 31) - kGridX) / Hkv && Hkv < 65536, "prefill_attention: grid too large");
+  const int64_t wgs = B * nt * Hkv;
+  const dim3 grid((unsigned)(wgs < kGridX ? wgs : kGridX), (unsigned)((wgs + kGridX - 1) / kGridX));
   const float sl2 = scale * 1.4426950408889634f;
   hipStream_t st = (hipStream_t)stream;
 #define LFS_PF(DD, PG)                                                                                             \

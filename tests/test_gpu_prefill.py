@@ -265,6 +265,21 @@ def test_prefill_ragged_work_items(Hq, Hkv, D, B, BS, scale):
     assert_close(f64(o), ref, f"work items Hq={Hq} Hkv={Hkv} D={D} B={B} BS={BS}")
 
 
+@pytest.mark.parametrize("max_q", [(1 << 20) - 100, 1 << 20])
+def test_prefill_many_empty_workgroups(max_q):
+    """Short prompts under a max_seqlen_q whose grid passes 2^20 workgroups
+    (several grid rows) and 2^32 threads."""
+    rng = np.random.default_rng(max_q)
+    B, Hq, Hkv, D = 64, 32, 8, 64
+    lens = rng.integers(1, 9, B)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=DEV)
+    q, k, v = (bf16(rng, int(lens.sum()), h, D) for h in (Hq, Hkv, Hkv))
+    o = K.flash_attn_varlen_func(q, k, v, cu, cu, max_q, max_q, 0.125)
+    assert torch.equal(o, K.flash_attn_varlen_func(q, k, v, cu, cu, 8, 8, 0.125))
+    c = cu.cpu().numpy()
+    assert_close(f64(o), P.prefill_attention(f64(q), f64(k), f64(v), c, c, 0.125), f"max_seqlen_q {max_q}")
+
+
 def test_prefill_argument_errors():
     q = torch.zeros(4, 8, 64, dtype=torch.bfloat16, device=DEV)
     kv = torch.zeros(4, 2, 64, dtype=torch.bfloat16, device=DEV)
