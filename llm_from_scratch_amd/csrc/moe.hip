@@ -184,7 +184,10 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_place_kernel(
 // workgroup per token left 160 of 256 threads idle at d = 768 and held them
 // at a barrier for the token's entries).  The entries of a token are the same
 // addresses in all its lanes.  KK > 0: kk at compile time, so that all rows
-// and down biases are loaded before the first sum.
+// and down biases are loaded before the first sum.  Workgroups in grid rows
+// of kCombineGridX: a launch takes less than 2^32 threads in x, and T * d / 8
+// may be more.
+constexpr int64_t kCombineGridX = 1 << 16;
 template <typename OutT, int KK>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const OutT* __restrict__ out, int64_t ld,
                                                           const int32_t* __restrict__ entry_row,
@@ -192,7 +195,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const OutT* __restrict
                                                           const float* __restrict__ topk_w, int top_k, int E,
                                                           int S, const float* __restrict__ b2, int d,
                                                           uint16_t* __restrict__ y, int64_t units) {
-  const int64_t u = blockIdx.x * 256ll + threadIdx.x;
+  const int64_t u = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
   if (u >= units) return;
   const int cpr = d / 8, kk = KK > 0 ? KK : top_k + S;
   const int64_t t = units >> 31 ? u / cpr : (int64_t)((unsigned)u / (unsigned)cpr);
@@ -441,10 +444,11 @@ extern "C" int lfs_moe_combine(const void* out, int32_t out_is_f32, int64_t ld, 
   LFS_REQUIRE(out && entry_row && topk_idx && topk_weight && y, "moe_combine: null pointer");
   LFS_REQUIRE((((uintptr_t)out) | ((uintptr_t)y)) % 16 == 0, "moe_combine: buffers must be 16-byte aligned");
   LFS_REQUIRE(T < (1ll << 31), "moe_combine: too many tokens");
-  const int64_t units = T * (d / 8);
+  const int64_t units = T * (d / 8), wgs = (units + 255) / 256;
+  const dim3 grid((unsigned)std::min(wgs, kCombineGridX), (unsigned)((wgs + kCombineGridX - 1) / kCombineGridX));
 #define LFS_MC(OT, KK)                                                                                              \
-  hipLaunchKernelGGL((moe_combine_kernel<OT, KK>), dim3((unsigned)((units + 255) / 256)), dim3(256), 0,              \
-                     (hipStream_t)stream, (const OT*)out, ld, entry_row, topk_idx, topk_weight, top_k, num_experts, \
+  hipLaunchKernelGGL((moe_combine_kernel<OT, KK>), grid, dim3(256), 0, (hipStream_t)stream,                         \
+                     (const OT*)out, ld, entry_row, topk_idx, topk_weight, top_k, num_experts, \
                      num_shared, down_bias, d, (uint16_t*)y, units)
 #define LFS_MCK(OT)                  \
   switch (top_k + num_shared) {      \

@@ -274,3 +274,18 @@ def test_moe_combine_entry_counts(k, S, d):
             ref = MO.moe_combine(out.double().cpu().numpy(), er, idx, w, E, S, np.zeros_like(b2) if bias is None else b2)
             # one bf16 rounding of an fp32 sum vs of a float64 sum
             assert np.all(np.abs(y.float().cpu().numpy() - ref) <= 2.0 ** -7 * np.abs(ref) + 1e-6)
+
+
+@pytest.mark.parametrize("T", [8191, 8192, 20001])
+def test_moe_combine_grid_rows(T):
+    """2^24 and more 8-column units (several grid rows, the last one part):
+    each row the fp32 sum of its two entries' rows, as torch has it."""
+    d, k, E = 16384, 2, 4
+    g = torch.Generator(device=DEV).manual_seed(T)
+    out = torch.randn(64, d, generator=g, device=DEV).to(torch.bfloat16)
+    rows = torch.randint(0, 64, (T, k), generator=g, device=DEV, dtype=torch.int32)
+    idx = torch.randint(0, E, (T, k), generator=g, device=DEV)
+    y = K.moe_combine(out, rows, idx, torch.rand(T, k, generator=g, device=DEV), E)
+    for t in range(0, T, 4096):
+        a, b = (out[rows[t:t + 4096, j].long()].float() for j in range(2))
+        assert torch.equal(y[t:t + 4096], (a + b).to(torch.bfloat16)), t
