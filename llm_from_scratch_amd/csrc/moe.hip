@@ -20,6 +20,7 @@
 //                    scans and places the entries per token, then sums each
 //                    segment in increasing entry order.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -33,18 +34,21 @@ constexpr int kTile = 128;  // rows per grouped-GEMM tile
 // Entry i = t * kk + j of the (token, pick) list, kk = top_k + S: picks
 // j < top_k are routed expert topk_idx[t, j] with weight topk_w[t, j]; the
 // rest are the shared experts E + (j - top_k) with weight 1.
-__device__ __forceinline__ void entry(const int64_t* idx, const float* w, int64_t i, int kk, int top_k, int E,
-                                      int& t, int& e, float& wt) {
-  t = (int)(i / kk);
-  const int j = (int)(i - (int64_t)t * kk);
+__device__ __forceinline__ void pick(const int64_t* idx, const float* w, int64_t t, int j, int top_k, int E, int& e,
+                                     float& wt) {
   if (j < top_k) {
-    const int64_t v = idx[(int64_t)t * top_k + j];
+    const int64_t v = idx[t * top_k + j];
     e = (v >= 0 && v < E) ? (int)v : -1;  // out-of-range picks are dropped
-    wt = w[(int64_t)t * top_k + j];
+    wt = w[t * top_k + j];
   } else {
     e = E + (j - top_k);
     wt = 1.0f;
   }
+}
+__device__ __forceinline__ void entry(const int64_t* idx, const float* w, int64_t i, int kk, int top_k, int E,
+                                      int& t, int& e, float& wt) {
+  t = (int)(i / kk);
+  pick(idx, w, t, (int)(i - (int64_t)t * kk), top_k, E, e, wt);
 }
 
 // moe_align in three launches over chunks of 1024 entries (workspace:
@@ -183,11 +187,24 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_place_kernel(
 // pairs numbered through, so that every lane has work whatever d is (one
 // workgroup per token left 160 of 256 threads idle at d = 768 and held them
 // at a barrier for the token's entries).  The entries of a token are the same
-// addresses in all its lanes.  KK > 0: kk at compile time, so that all rows
-// and down biases are loaded before the first sum.  Workgroups in grid rows
-// of kCombineGridX: a launch takes less than 2^32 threads in x, and T * d / 8
-// may be more.
+// addresses in all its lanes.
+//
+// Bound by the round trips of dependent loads (entries, then rows and down
+// biases) and, above some 4096 tokens, by the rows' bytes.  KK > 0, up to 10
+// entries (8 picks and 2 shared experts): kk at compile time, all entries,
+// then all rows and biases in flight at once, 12 registers (fp32 rows 16) per
+// entry.  KK == 0, more entries: four at a time, in two passes (the sum takes
+// all rows first), the workgroup's entries in LDS, as loading them again per
+// group and lane is half of the address work.  Workgroup per token -> this,
+// d 768, bf16, with biases: 300 tokens, 3 entries 3.8 -> 2.8 us, 4 4.3 -> 3.1,
+// 9 6.5 -> 4.1, 17 10.1 -> 8.4; 2048 tokens 4.8 -> 3.8, 5.4 -> 4.3, 10.2 ->
+// 7.7, 17.2 -> 16.1; 16384 tokens 28.6 -> 17.8, 34.2 -> 21.9, 63 -> 50, 147 ->
+// 113.
+//
+// Workgroups in grid rows of kCombineGridX: a launch takes less than 2^32
+// threads in x, and T * d / 8 may be more.
 constexpr int64_t kCombineGridX = 1 << 16;
+constexpr int kCombineStage = 1024;  // entries in LDS: any count from d = 256 up
 template <typename OutT, int KK>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const OutT* __restrict__ out, int64_t ld,
                                                           const int32_t* __restrict__ entry_row,
@@ -195,58 +212,126 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const OutT* __restrict
                                                           const float* __restrict__ topk_w, int top_k, int E,
                                                           int S, const float* __restrict__ b2, int d,
                                                           uint16_t* __restrict__ y, int64_t units) {
-  const int64_t u = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
-  if (u >= units) return;
+  const int64_t u0 = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 256, u = u0 + threadIdx.x;
   const int cpr = d / 8, kk = KK > 0 ? KK : top_k + S;
-  const int64_t t = units >> 31 ? u / cpr : (int64_t)((unsigned)u / (unsigned)cpr);
+  auto token = [&](int64_t x) -> int64_t {
+    return units >> 31 ? x / cpr : (int64_t)((unsigned)x / (unsigned)cpr);
+  };
+  // KK == 0: the workgroup's tokens' entries in LDS, where they fit
+  __shared__ int srow[KK > 0 ? 1 : kCombineStage], sex[KK > 0 ? 1 : kCombineStage];
+  __shared__ float swt[KK > 0 ? 1 : kCombineStage];
+  int64_t t0 = 0;
+  bool staged = false;
+  if constexpr (KK == 0) {
+    t0 = token(min(u0, units - 1));
+    const int n = (int)min(token(min(u0 + 255, units - 1)) - t0 + 1, (int64_t)kCombineStage) * kk;
+    staged = n <= kCombineStage;
+    if (staged) {
+      for (int i = threadIdx.x; i < n; i += 256) {
+        srow[i] = entry_row[t0 * kk + i];
+        pick(topk_idx, topk_w, t0 + i / kk, i % kk, top_k, E, sex[i], swt[i]);
+      }
+      __syncthreads();
+    }
+  }
+  if (u >= units) return;
+  const int64_t t = token(u);
   const int c = (int)(u - t * cpr) * 8;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  auto add_row = [&](int row) {
-    float v[8];
-    if constexpr (sizeof(OutT) == 4) {
-      const float4* p = reinterpret_cast<const float4*>(out + (int64_t)row * ld + c);
-      const float4 a = p[0], b = p[1];
-      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    } else {
-      unpack8(*reinterpret_cast<const uint4*>(out + (int64_t)row * ld + c), v);
-    }
+  constexpr int U = KK > 0 ? KK : 4;  // entries at once
+  typedef std::conditional_t<sizeof(OutT) == 4, float4, uint4> V;
+  constexpr int NV = sizeof(OutT) == 4 ? 2 : 1;
+  int row[U], ex[U];
+  float wt[U], bb[U][8];
+  V r[U][NV];
+  const int at = staged ? (int)(t - t0) * kk : 0;
+  // Entries j0 .. j0 + U - 1.  Absent and dropped ones load no row and
+  // add 0, which leaves acc, never -0, as it is.
+  auto load_entries = [&](int j0) {
 #pragma unroll
-    for (int x = 0; x < 8; ++x) acc[x] += v[x];
+    for (int j = 0; j < U; ++j)
+      row[j] = KK == 0 && j0 + j >= kk ? -1 : staged ? srow[at + j0 + j] : entry_row[t * kk + j0 + j];
   };
-  auto add_bias = [&](int e, float wt) {
-    const float* bb = b2 + (int64_t)e * d + c;
+  auto load_picks = [&](int j0) {
 #pragma unroll
-    for (int x = 0; x < 8; ++x) acc[x] = fmaf(wt, bb[x], acc[x]);
+    for (int j = 0; j < U; ++j) {
+      const int i = min(j0 + j, kk - 1);
+      if (staged) ex[j] = sex[at + i], wt[j] = swt[at + i];
+      else pick(topk_idx, topk_w, t, i, top_k, E, ex[j], wt[j]);
+    }
+  };
+  auto load_rows = [&] {
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+      for (int x = 0; x < NV; ++x) {
+        r[j][x] = V{};
+        if (row[j] >= 0) r[j][x] = reinterpret_cast<const V*>(out + (int64_t)row[j] * ld + c)[x];
+      }
+  };
+  auto load_biases = [&] {
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+      for (int x = 0; x < 8; ++x) bb[j][x] = b2[(int64_t)max(ex[j], 0) * d + c + x];
+  };
+  auto add_rows = [&] {
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      float v[8];
+      if constexpr (NV == 2) {
+        v[0] = r[j][0].x; v[1] = r[j][0].y; v[2] = r[j][0].z; v[3] = r[j][0].w;
+        v[4] = r[j][1].x; v[5] = r[j][1].y; v[6] = r[j][1].z; v[7] = r[j][1].w;
+      } else {
+        unpack8(r[j][0], v);
+      }
+#pragma unroll
+      for (int x = 0; x < 8; ++x) acc[x] += v[x];
+    }
+  };
+  auto add_biases = [&](const int (&row)[U], const float (&wt)[U]) {
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+      for (int x = 0; x < 8; ++x) acc[x] = row[j] >= 0 ? fmaf(wt[j], bb[j][x], acc[x]) : acc[x];
   };
   if constexpr (KK > 0) {
-    int row[KK], ex[KK];
-    float wt[KK];
-#pragma unroll
-    for (int j = 0; j < KK; ++j) {
-      int tt;
-      entry(topk_idx, topk_w, t * KK + j, KK, top_k, E, tt, ex[j], wt[j]);
-      row[j] = entry_row[t * KK + j];
-    }
-#pragma unroll
-    for (int j = 0; j < KK; ++j)
-      if (row[j] >= 0) add_row(row[j]);
+    load_entries(0);
     if (b2 != nullptr) {
-#pragma unroll
-      for (int j = 0; j < KK; ++j)
-        if (row[j] >= 0) add_bias(ex[j], wt[j]);
+      load_picks(0);
+      load_rows();
+      load_biases();
+      add_rows();
+      add_biases(row, wt);
+    } else {
+      load_rows();
+      add_rows();
     }
   } else {
-    for (int j = 0; j < kk; ++j) {
-      const int row = entry_row[t * kk + j];
-      if (row >= 0) add_row(row);
+    // four at a time, the next four's entries loaded with their values
+    int now[U];
+    auto take = [&](int j) {  // entries j .. j + U - 1 out of row, the next ones on their way into it
+#pragma unroll
+      for (int i = 0; i < U; ++i) now[i] = row[i];
+      if (j + U < kk) load_entries(j + U);
+    };
+    load_entries(0);
+    for (int j = 0; j < kk; j += U) {
+      load_rows();
+      take(j);
+      add_rows();
     }
     if (b2 != nullptr) {
-      for (int j = 0; j < kk; ++j) {
-        if (entry_row[t * kk + j] < 0) continue;
-        int tt, e;
-        float wt;
-        entry(topk_idx, topk_w, t * kk + j, kk, top_k, E, tt, e, wt);
-        add_bias(e, wt);
+      load_entries(0);
+      load_picks(0);
+      for (int j = 0; j < kk; j += U) {
+        float w[U];
+        load_biases();
+        take(j);
+#pragma unroll
+        for (int i = 0; i < U; ++i) w[i] = wt[i];
+        if (j + U < kk) load_picks(j + U);
+        add_biases(now, w);
       }
     }
   }
@@ -452,9 +537,16 @@ extern "C" int lfs_moe_combine(const void* out, int32_t out_is_f32, int64_t ld, 
                      num_shared, down_bias, d, (uint16_t*)y, units)
 #define LFS_MCK(OT)                  \
   switch (top_k + num_shared) {      \
+    case 1: LFS_MC(OT, 1); break;    \
     case 2: LFS_MC(OT, 2); break;    \
     case 3: LFS_MC(OT, 3); break;    \
+    case 4: LFS_MC(OT, 4); break;    \
     case 5: LFS_MC(OT, 5); break;    \
+    case 6: LFS_MC(OT, 6); break;    \
+    case 7: LFS_MC(OT, 7); break;    \
+    case 8: LFS_MC(OT, 8); break;    \
+    case 9: LFS_MC(OT, 9); break;    \
+    case 10: LFS_MC(OT, 10); break;  \
     default: LFS_MC(OT, 0); break;   \
   }
   if (out_is_f32) {

@@ -15,6 +15,8 @@ Cases: cfg5's 8 experts top-2 + 1 shared, 64 experts top-6, token counts
 across tile edges (1, 127, 128, 129, 1000), dropped (-1 / out-of-range)
 picks, strided per-expert weight views, bf16 and fp32 inputs.
 """
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -274,6 +276,38 @@ def test_moe_combine_entry_counts(k, S, d):
             ref = MO.moe_combine(out.double().cpu().numpy(), er, idx, w, E, S, np.zeros_like(b2) if bias is None else b2)
             # one bf16 rounding of an fp32 sum vs of a float64 sum
             assert np.all(np.abs(y.float().cpu().numpy() - ref) <= 2.0 ** -7 * np.abs(ref) + 1e-6)
+
+
+@pytest.mark.parametrize("k,S,d", [(1, 0, 24), (3, 1, 768), (6, 0, 16), (6, 1, 136), (6, 2, 136), (8, 1, 1024),
+                                   (8, 2, 24), (8, 3, 768), (8, 4, 8), (17, 0, 256), (40, 8, 2048), (30, 2, 40)])
+def test_moe_combine_any_entry_count(k, S, d):
+    """Every compiled entry count (to 10) and the general loop, its entries in
+    LDS or, where a workgroup's tokens have too many (d = 8, 40), not: the
+    rows' sum in entry order, bit for bit; with biases within the fp32 sums'
+    bound and one bf16 rounding.  Dropped picks, and nothing but these."""
+    rng = np.random.default_rng(k * 10 + S)
+    T, E = 137, max(8, k)
+    idx, w = picks(rng, T, E, k, bad=9)
+    er = MO.moe_align(idx, w, E, S)[3]
+    rows = K.moe_align(dev(idx), dev(w), E, S)
+    assert np.array_equal(rows.entry_row.cpu().numpy(), er)
+    b2 = rng.standard_normal((E + S, d)).astype(np.float32)
+    for dt in (torch.bfloat16, torch.float32):
+        out = dev(rng.standard_normal((rows.num_rows, d)).astype(np.float32)).to(dt)
+        y = K.moe_combine(out, rows.entry_row, dev(idx), dev(w), E, S)
+        acc = torch.zeros(T, d, device=DEV)
+        for j in range(k + S):
+            r = rows.entry_row[:, j].long()
+            acc += torch.where((r >= 0)[:, None], out[r.clamp_min(0)].float(), 0)
+        assert torch.equal(y, acc.to(torch.bfloat16))
+        y = K.moe_combine(out, rows.entry_row, dev(idx), dev(w), E, S, dev(b2)).double().cpu().numpy()
+        o = out.double().cpu().numpy()
+        ref, size = MO.moe_combine(o, er, idx, w, E, S, b2), MO.moe_combine(np.abs(o), er, idx, w, E, S, np.abs(b2))
+        # 2(k + S) roundings of at most 2^-24 of the sum's terms, then both sides' rounding to
+        # bf16, each half an ulp of 2^-7 of a value whose significand is 1
+        assert (np.abs(y - ref) <= 2.0 ** -7 * np.abs(ref) + 2 * (k + S) * 2.0 ** -24 * size).all()
+    none = torch.full((T, k + S), -1, dtype=torch.int32, device=DEV)
+    assert not K.moe_combine(torch.full_like(out[:1], math.nan), none, dev(idx), dev(w), E, S, dev(b2)).any()
 
 
 @pytest.mark.parametrize("T", [8191, 8192, 20001])
