@@ -491,15 +491,15 @@ __global__ __launch_bounds__(64 * kRouteTokens) void moe_route_kernel(
 }
 
 // Large batches in index form (the grouped dispatch: no routed bias), E <= EP
-// = 8, 16 or 32 experts: a wave takes 32 / EP tokens, so that each gate row
+// = 4, 8, 16 or 32 experts: a wave takes 32 / EP tokens, so that each gate row
 // chunk is unpacked once for them and the tokens' memory round trips overlap.
 // Their 32 logits are summed by halving: at lane distance 32, 16, 8, 4, 2 a
 // lane hands half of its sums over and keeps the others, the pairs and order
 // of the butterfly (the same bits) in 31 additions instead of 192, and
 // lane bits 5..1 end as (token, expert).  Each group of 2 * EP lanes then
-// picks its token's top k.  16384 tokens, d 768, 8 experts: 39 -> 13 us
-// against a wave per token, which waits out its loads, its eight butterflies
-// and its picks one after the other.
+// picks its token's top k.  Device time, 16384 tokens, d 768, 8 experts: 32
+// -> 9-10 us against a wave per token, which waits out its loads, its eight
+// butterflies and its picks one after the other.
 template <int EP>
 __global__ __launch_bounds__(256) void moe_route_rows_kernel(const uint16_t* __restrict__ h,
                                                              const uint16_t* __restrict__ gw,
@@ -509,7 +509,7 @@ __global__ __launch_bounds__(256) void moe_route_rows_kernel(const uint16_t* __r
                                                              float* __restrict__ topk_w) {
   constexpr int TW = 32 / EP;  // tokens per wave
   const int lane = threadIdx.x & 63;
-  const int64_t t0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * TW;
+  const int64_t t0 = ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * TW;
   if (t0 >= T) return;
   const int cpr = d / 8;
   float acc[32];  // token, expert
@@ -569,7 +569,7 @@ __global__ __launch_bounds__(256) void moe_route_rows_kernel(const uint16_t* __r
     };
     if constexpr (EP > 16) step(std::integral_constant<int, 32>{});
     if constexpr (EP > 8) step(std::integral_constant<int, 16>{});
-    step(std::integral_constant<int, 8>{});
+    if constexpr (EP > 4) step(std::integral_constant<int, 8>{});
     step(std::integral_constant<int, 4>{});
     step(std::integral_constant<int, 2>{});
     if (e == bi) { chosen = true; myk = k; }
@@ -593,6 +593,24 @@ __global__ __launch_bounds__(256) void moe_route_rows_kernel(const uint16_t* __r
     topk_w[t * top_k + myk] = wgt;
   }
 }
+
+// Tokens from which that form is taken.  Fewer tokens leave it fewer waves than
+// the chip has SIMDs, each walking d alone, where the wave per token has 32 /
+// EP times as many: with few experts or wide rows it is then the slower one.
+// Wave per token against this, us: 8 experts, 2048 tokens, d 1024 6.9 / 6.7,
+// d 2048 9.5 / 10.2, 4096 tokens 17.1 / 10.6; 16 experts, 2048 tokens, d 2048
+// 15.8 / 15.2, d 4096 26.6 / 27.1, 4096 tokens 52.5 / 43.2; 4 experts, 3000
+// tokens, d 768 5.1 / 6.1, 4096 tokens 7.4 / 6.1, of d 4096 18.9 / 21.1; 32
+// experts, 1025 tokens, d 4096 50.4 / 45.4.
+inline int64_t route_rows_tokens(int E, int d) {
+  if (E <= 4) return d <= 1024 ? 4096 : 8192;
+  return d > (E <= 8 ? 1024 : E <= 16 ? 2048 : 1 << 30) ? 4096 : 0;
+}
+// Up to here a wave is a workgroup of its own, so that each gets a SIMD (2048
+// tokens of 4096, 8 experts: 26.1 us in workgroups of four, 17.4); more waves
+// go in groups of four (16384 tokens of 768, 2 experts: 9.3 us alone, 6.9; 8
+// experts the same).
+constexpr int64_t kRouteWaves = 1024;
 
 // Small batches (decode): one workgroup of 4 waves per token, so that the
 // tokens spread over as many CUs as possible.
@@ -995,12 +1013,17 @@ extern "C" int lfs_moe_route(const void* h, const void* gate_weight, const float
     hipLaunchKernelGGL(moe_route_token_kernel, dim3((unsigned)T), dim3(256), 0, (hipStream_t)stream,
                        (const uint16_t*)h, (const uint16_t*)gate_weight, expert_bias, down_bias, dense_weights,
                        bias_out, d, num_experts, num_shared, top_k, topk_idx, topk_weight);
-  else if (bias_out == nullptr && num_experts <= 32) {
+  else if (bias_out == nullptr && num_experts <= 32 && T >= route_rows_tokens(num_experts, d)) {
 #define LFS_RR(EP)                                                                                                   \
-  hipLaunchKernelGGL(moe_route_rows_kernel<EP>, dim3((unsigned)((T + 128 / EP - 1) / (128 / EP))), dim3(256), 0,      \
-                     (hipStream_t)stream, (const uint16_t*)h, (const uint16_t*)gate_weight, expert_bias, dense_weights, \
-                     T, d, num_experts, num_shared, top_k, topk_idx, topk_weight)
-    if (num_experts <= 8) LFS_RR(8);
+  do {                                                                                                               \
+    const int64_t waves = (T + 32 / EP - 1) / (32 / EP);                                                              \
+    const int wpg = waves <= kRouteWaves ? 1 : 4; /* waves per workgroup */                                          \
+    hipLaunchKernelGGL(moe_route_rows_kernel<EP>, dim3((unsigned)((waves + wpg - 1) / wpg)), dim3(64 * wpg), 0,        \
+                       (hipStream_t)stream, (const uint16_t*)h, (const uint16_t*)gate_weight, expert_bias,            \
+                       dense_weights, T, d, num_experts, num_shared, top_k, topk_idx, topk_weight);                  \
+  } while (0)
+    if (num_experts <= 4) LFS_RR(4);
+    else if (num_experts <= 8) LFS_RR(8);
     else if (num_experts <= 16) LFS_RR(16);
     else LFS_RR(32);
 #undef LFS_RR

@@ -237,6 +237,24 @@ def test_moe_route_index_form_large_batch_same_bits(E, S, k, d):
     assert torch.equal(only[2], res[2]) and torch.equal(only[3], res[3])
 
 
+@pytest.mark.parametrize("E,S,k,d,T", [(4, 1, 1, 768, 4099), (3, 0, 2, 520, 4096), (1, 0, 1, 2048, 8197), (2, 2, 2, 64, 33000),
+                                       (8, 1, 2, 2048, 4097), (7, 1, 3, 768, 16399), (16, 1, 4, 4096, 4099),
+                                       (5, 0, 2, 2048, 2000)])
+def test_moe_route_rows_sizes_same_bits(E, S, k, d, T):
+    """The gate without the routed bias at the sizes where its form and its
+    waves per workgroup change (4 experts and fewer, wide rows, more waves than
+    SIMDs), against the kernel of a workgroup per token on slices."""
+    g = torch.Generator(device=DEV).manual_seed(E * 100 + T)
+    h = torch.randn(T, d, generator=g, device=DEV).to(torch.bfloat16)
+    h[::50] = 0
+    gate = (torch.randn(E, d, generator=g, device=DEV) / d ** 0.5).to(torch.bfloat16)
+    bias = torch.randn(E, generator=g, device=DEV) * 0.01
+    res = K.moe_route(h, gate, bias, None, k, S, return_topk=True)
+    parts = [K.moe_route(h[i:i + 1000], gate, bias, None, k, S, return_topk=True) for i in range(0, T, 1000)]
+    for got, want in zip((res[0], res[2], res[3]), zip(*[(p[0], p[2], p[3]) for p in parts])):
+        assert torch.equal(got, torch.cat(want))
+
+
 @pytest.mark.parametrize("E,k", [(8, 2), (16, 4), (32, 4)])
 def test_moe_route_nan_gate_same_weights(E, k):
     """NaN in a gate row or in the selection bias (one expert, the first or
