@@ -124,70 +124,88 @@ __device__ __forceinline__ int vswz(int r) {
   return D == 64 ? ((r >> 1) & 1) << 2 : (r & 3) << 2;
 }
 
-// Row tile `tile` of sequence i that comes at place `rank` when all tiles of R
-// rows are ordered by the number of KT-key tiles they walk, longest first.  A
-// launch fills the chip in id order and deals ids to the shader engines in
-// turn, so ids in any other order leave engines or the tail idle (six cached
-// prompts of 700-6000 tokens: 700 us with the sequences interleaved tile by
-// tile, 551 us ranked).  With B <= 64 sequences lane s holds sequence s, and
-// the lanes test 64 thresholds at once: n_s(c) tiles of sequence s walk at
-// least c key tiles, and N(c) = sum n_s(c) > rank holds up to the tile's own
-// count.  False (nothing set) for larger batches, whose many sequences even
-// out, and for contexts whose arithmetic would not fit; tile is -1 past the
-// last.
+// x / v.d for x < 2^31, by the reciprocal that div_by() rounded up: the product's
+// high word is the quotient or one more.
+struct Div {
+  unsigned d, inv;
+};
+inline Div div_by(unsigned d) { return Div{d, d == 1 ? 0u : (unsigned)((0xFFFFFFFFull + d) / d)}; }
+__device__ __forceinline__ unsigned operator/(unsigned x, Div v) {
+  const unsigned q = v.inv != 0 ? __umulhi(x, v.inv) : x;
+  return q * v.d > x ? q - 1 : q;
+}
+
+// Inclusive sum over the wave's lanes.
+__device__ __forceinline__ int scan_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast 15: rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast 31: rows 2 and 3
+  return v;
+}
+
+// A sequence's first query row and token, and their numbers.
+struct Seq {
+  int q0, lq, k0, lk;
+};
+
+// Row tile `tile` of sequence `seq` (the i-th) that comes at place `rank` when
+// all tiles of R rows are ordered by the number of KT-key tiles they walk,
+// longest first.  A launch fills the chip in id order and deals ids to the
+// shader engines in turn, so ids in any other order leave engines or the tail
+// idle (six cached prompts of 700-6000 tokens: 700 us with the sequences
+// interleaved tile by tile, 551 us ranked).  With B <= 64 sequences lane s
+// holds sequence s; N(c), the tiles that walk at least c key tiles, is one sum
+// over the wave, and a binary search finds the largest c with N(c) > rank: the
+// same few hundred cycles for any B (testing 64 thresholds a pass, each a loop
+// over B, took 0.2 us per sequence from every workgroup, also from the empty
+// ones of a ragged batch, which now leave after the first sum).  False (nothing
+// set) for larger batches, whose many sequences even out, and for contexts
+// whose arithmetic would not fit; tile is -1 past the last.
 template <int R>
-__device__ __forceinline__ bool ranked_item(const int32_t* cu_q, const int32_t* cu_k, int B, int G, int rtiles,
-                                            int rank, int& i, int& tile) {
+__device__ __forceinline__ bool ranked_item(const int32_t* cu_q, const int32_t* cu_k, int B, Div G, int rtiles,
+                                            int rank, int& i, int& tile, Seq& seq) {
   if (B > 64) return false;
   const int lane = threadIdx.x & 63;
-  int nt = 0, off = 0, most = 0;
+  int q0 = 0, lq = 0, k0 = 0, lk = 0, nt = 0, off = 0, most = 0;
   if (lane < B) {
-    const int lq = cu_q[lane + 1] - cu_q[lane], lk = cu_k[lane + 1] - cu_k[lane];
+    q0 = cu_q[lane], lq = cu_q[lane + 1] - q0;
+    k0 = cu_k[lane], lk = cu_k[lane + 1] - k0;
+    off = lk - lq;
     if (lq > 0) {
-      off = lk - lq;
-      const int64_t tiles = ((int64_t)lq * G + R - 1) / R;
-      const int64_t end = off + (tiles * R - 1) / G + 1;  // keys of the last tile (its full rows)
-      nt = (int)min(tiles, (int64_t)rtiles);
-      most = off < 0 || end > (1 << 26) ? 1 << 30 : (int)((end + KT - 1) / KT);
+      if (off < 0 || lk > 1 << 26) {
+        most = 1 << 30;
+      } else {
+        const unsigned tiles = ((unsigned)lq * G.d + R - 1) / R;
+        nt = min((int)tiles, rtiles);
+        most = (off + (int)((tiles * R - 1) / G) + KT) / KT;  // key tiles of the last tile (its full rows)
+      }
     }
   }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) most = max(most, __shfl_xor(most, d, 64));
-  most = __builtin_amdgcn_readfirstlane(most);
-  if (most >= 1 << 30) return false;
-  // tiles of sequence s that walk at least c >= 1 key tiles
-  auto count = [&](int s, int c) {
-    const int n = __builtin_amdgcn_readlane(nt, s);
-    return max(0, n - max(0, G * (KT * (c - 1) - __builtin_amdgcn_readlane(off, s)) / R));
-  };
-  auto total = [&](int c) {
-    int n = 0;
-    for (int s = 0; s < B; ++s) n += count(s, c);
-    return n;
-  };
-  int lo = 1, range = most;  // the tile's count is in [lo, lo + range)
+  if (__any(most >= 1 << 30)) return false;
+  // tiles of the lane's sequence that walk at least c >= 1 key tiles, and of all
+  auto count = [&](int c) { return max(0, nt - max(0, (int)G.d * (KT * (c - 1) - off)) / R); };
+  auto total = [&](int c) { return __builtin_amdgcn_readlane(scan_sum(count(c)), 63); };
   tile = -1;
   i = 0;
-  while (true) {
-    const int step = max((range + 63) / 64, 1);
-    const int k = __popcll(__ballot(total(lo + lane * step) > rank));
-    if (k == 0) return true;  // past the last tile (only at lo = 1)
-    lo += (k - 1) * step;
-    if (step == 1) break;
-    range = step;
+  int tlo = total(1), thi = 0;
+  if (tlo <= rank) return true;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) most = max(most, __shfl_xor(most, d, 64));
+  int lo = 1, hi = __builtin_amdgcn_readfirstlane(most) + 1;  // N(lo) > rank >= N(hi) = thi
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1, n = total(mid);
+    if (n > rank) lo = mid;
+    else hi = mid, thi = n;
   }
-  rank -= total(lo + 1);
-  for (int s = 0; s < B; ++s) {
-    const int n = count(s, lo), m = n - count(s, lo + 1);
-    if (rank < m) {
-      i = s;
-      tile = __builtin_amdgcn_readlane(nt, s) - n + rank;
-      break;
-    }
-    rank -= m;
-  }
-  i = __builtin_amdgcn_readfirstlane(i);
-  tile = __builtin_amdgcn_readfirstlane(tile);
+  rank -= thi;
+  const int n = count(lo), m = n - count(hi), incl = scan_sum(m);
+  i = __builtin_ctzll(__ballot(incl > rank));
+  tile = __builtin_amdgcn_readlane(nt - n - incl + m, i) + rank;
+  seq.q0 = __builtin_amdgcn_readlane(q0, i), seq.lq = __builtin_amdgcn_readlane(lq, i);
+  seq.k0 = __builtin_amdgcn_readlane(k0, i), seq.lk = __builtin_amdgcn_readlane(lk, i);
   return true;
 }
 
@@ -195,8 +213,8 @@ template <int D, bool PAGED>
 __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k, const int32_t* __restrict__ bt,
-    int64_t bt_stride, int BS, int64_t num_slots, uint16_t* __restrict__ out, int B, int Hkv, int G, int rtiles,
-    int xsplit, float scale_log2) {
+    int64_t bt_stride, int64_t num_slots, uint16_t* __restrict__ out, Div dB, Div dHkv, Div G, Div dBS,
+    int rtiles, int xshift, float scale_log2) {
   constexpr int NDC = D / 16;            // 16-dim MFMA k steps of S
   constexpr int NDB = D / 32;            // 32-dim blocks of O^T
   constexpr int RB = 2 * D;              // bytes of a tile row
@@ -208,35 +226,41 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
   static_assert(RPW <= 16 && RPW == NC * RPC, "a wave copies rows of one 16-key half");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[4 * TB];  // K0, K1, V0, V1
 
+  const int B = (int)dB.d, Hkv = (int)dHkv.d, BS = (int)dBS.d;
   // Work item of this workgroup.  Workgroup ids are dealt round-robin to the
-  // 8 XCDs: XCD x takes kv head x / xsplit (xsplit = 8 / Hkv where Hkv divides
-  // 8: every xsplit-th row tile of it), so that a pair's K and V are read
-  // through one or few L2s and ragged sequences still load the XCDs evenly.
+  // 8 XCDs: XCD x takes kv head x >> xshift (2^xshift = 8 / Hkv where Hkv
+  // divides 8: every 2^xshift-th row tile of it), so that a pair's K and V are
+  // read through one or few L2s and ragged sequences still load the XCDs
+  // evenly.
   int rank = blockIdx.y * gridDim.x + blockIdx.x, kh;
-  if (xsplit > 0) {
-    kh = (rank & 7) / xsplit;
-    rank = (rank >> 3) * xsplit + ((rank & 7) - kh * xsplit);
+  if (xshift >= 0) {
+    kh = (rank & 7) >> xshift;
+    rank = ((rank >> 3) << xshift) + ((rank & 7) - (kh << xshift));
   } else {
-    kh = rank % Hkv;
-    rank /= Hkv;
+    const int r = (int)((unsigned)rank / dHkv);
+    kh = rank - r * Hkv;
+    rank = r;
   }
   int i, tile;
-  if (!ranked_item<RW * NW>(cu_q, cu_k, B, G, rtiles, rank, i, tile)) {
-    i = rank % B;
-    tile = rtiles - 1 - rank / B;
+  Seq seq;
+  if (!ranked_item<RW * NW>(cu_q, cu_k, B, G, rtiles, rank, i, tile, seq)) {
+    const int r = (int)((unsigned)rank / dB);
+    i = rank - r * B;
+    tile = rtiles - 1 - r;
+    seq.q0 = cu_q[i], seq.lq = cu_q[i + 1] - seq.q0;
+    seq.k0 = cu_k[i], seq.lk = cu_k[i + 1] - seq.k0;
   }
-  const int q0 = cu_q[i], lq = cu_q[i + 1] - q0;
-  if (tile < 0 || (int64_t)tile * (RW * NW) >= (int64_t)lq * G) return;  // the whole workgroup
+  const int q0 = seq.q0, lq = seq.lq, k0 = seq.k0, lk = seq.lk;
+  if (tile < 0 || (int64_t)tile * (RW * NW) >= (int64_t)lq * G.d) return;  // the whole workgroup
   const unsigned r0 = (unsigned)tile * (RW * NW);  // its first row
-  const int k0 = cu_k[i], lk = cu_k[i + 1] - k0;
   const int off = lk - lq;                 // position of query token 0
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int c32 = lane & 31, h = lane >> 5;
-  const int Hq = Hkv * G;
-  const unsigned rows = (unsigned)lq * G;
+  const int Hq = Hkv * (int)G.d;
+  const unsigned rows = (unsigned)lq * G.d;
   // this lane's row; rows past the sequence are computed as its last row and not stored
   const unsigned row = r0 + RW * wave + c32;
-  const int tq = min(row, rows - 1) / G, hq = min(row, rows - 1) - tq * G;
+  const int tq = min(row, rows - 1) / G, hq = min(row, rows - 1) - tq * G.d;
   const int qp = off + tq;                 // its position
   // positions of the wave's first and last row, and of the workgroup's last
   const int pfirst = __builtin_amdgcn_readfirstlane(off + (int)(min(r0 + RW * wave, rows - 1) / G));
@@ -268,8 +292,9 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
   const int hoff = (RPW * wave) & ~15;  // the wave's half within a tile
   int blk = 0, boff = 0, lblk = 0, loff = 0;  // block and offset of the half's first key, and of key lk - 1
   if constexpr (PAGED) {
-    blk = hoff / BS, boff = hoff - blk * BS;
-    lblk = max(lk - 1, 0) / BS, loff = max(lk - 1, 0) - lblk * BS;
+    boff = hoff;
+    while (boff >= BS) boff -= BS, ++blk;
+    lblk = (int)((unsigned)max(lk - 1, 0) / dBS), loff = max(lk - 1, 0) - lblk * BS;
   }
   auto entry = [&](int t) -> int {  // table entry of the half that starts at key t
     int64_t e = (int64_t)i * bt_stride + min((int64_t)(t < lk ? blk : lblk), bt_stride - 1);
@@ -311,7 +336,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
   // Q^T (B operand): lane l supplies row l % 32, dims 16c + 8h .. +7
   v8bf qb[NDC];
   {
-    const uint16_t* qr = q + ((int64_t)(q0 + tq) * Hq + (int64_t)kh * G + hq) * D + 8 * h;
+    const uint16_t* qr = q + ((int64_t)(q0 + tq) * Hq + (int64_t)kh * G.d + hq) * D + 8 * h;
 #pragma unroll
     for (int c = 0; c < NDC; ++c) {
       qb[c] = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4*>(qr + 16 * c));
@@ -442,7 +467,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
   // ---- normalise and store: lane l holds row l % 32, dims 32db + 8i + 4h .. +3
   if (row < rows) {
     const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-    uint16_t* dst = out + ((int64_t)(q0 + tq) * Hq + (int64_t)kh * G + hq) * D + 4 * h;
+    uint16_t* dst = out + ((int64_t)(q0 + tq) * Hq + (int64_t)kh * G.d + hq) * D + 4 * h;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
@@ -480,18 +505,19 @@ extern "C" int lfs_prefill_attention(const void* q, const void* k, const void* v
   }
   const int G = Hq / Hkv;
   const int64_t rtiles = ((int64_t)max_seqlen_q * G + RW * NW - 1) / (RW * NW);
-  const int xsplit = Hkv <= 8 && 8 % Hkv == 0 ? 8 / Hkv : 0;
-  const int64_t nt = xsplit > 0 ? (rtiles + xsplit - 1) / xsplit * xsplit : rtiles;
+  const int xshift = Hkv <= 8 && 8 % Hkv == 0 ? __builtin_ctz(8 / Hkv) : -1;
+  const int64_t nt = xshift > 0 ? (rtiles + (1 << xshift) - 1) >> xshift << xshift : rtiles;
   LFS_REQUIRE(B * nt < ((1ll << 31) - kGridX) / Hkv && Hkv < 65536, "prefill_attention: grid too large");
   const int64_t wgs = B * nt * Hkv;
   const dim3 grid((unsigned)(wgs < kGridX ? wgs : kGridX), (unsigned)((wgs + kGridX - 1) / kGridX));
   const float sl2 = scale * 1.4426950408889634f;
   hipStream_t st = (hipStream_t)stream;
+  const Div dBS = div_by(block_tables != nullptr ? block_size : 1);
 #define LFS_PF(DD, PG)                                                                                             \
   hipLaunchKernelGGL((prefill_attention_kernel<DD, PG>), grid, dim3(64 * NW), 0, st, (const uint16_t*)q,        \
                      (const uint16_t*)k, (const uint16_t*)v, cu_seqlens_q, cu_seqlens_k, block_tables,             \
-                     PG ? bt_stride : 0, PG ? block_size : 0, num_slots, (uint16_t*)out, (int)B, Hkv, G,            \
-                     (int)rtiles, xsplit, sl2)
+                     PG ? bt_stride : 0, num_slots, (uint16_t*)out, div_by((unsigned)B), div_by(Hkv), div_by(G),   \
+                     dBS, (int)rtiles, xshift, sl2)
   if (block_tables != nullptr) {
     if (D == 64) LFS_PF(64, true);
     else LFS_PF(128, true);

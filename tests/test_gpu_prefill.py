@@ -265,6 +265,26 @@ def test_prefill_ragged_work_items(Hq, Hkv, D, B, BS, scale):
     assert_close(f64(o), ref, f"work items Hq={Hq} Hkv={Hkv} D={D} B={B} BS={BS}")
 
 
+@pytest.mark.parametrize("Hq,Hkv,D", [(12, 4, 64), (10, 2, 128), (3, 3, 64), (7, 1, 64)])
+def test_prefill_one_long_prompt_among_short(Hq, Hkv, D):
+    """A prompt of 2001 tokens beside 63 of 0-70 (most work items are past the
+    last tile; G and Hkv of 3, 5 and 7 divide by a rounded reciprocal), a batch
+    of equal prompts, and one prompt alone: every sequence the same bits as by
+    itself in index order (beside 64 empty ones, which the search passes by)."""
+    rng = np.random.default_rng(Hq)
+    long = [2001 if b == 40 else (7 * b) % 71 for b in range(64)]
+    for lens in (long, [33] * 64, [130]):
+        cu = np.concatenate([[0], np.cumsum(lens)])
+        q, k, v = (bf16(rng, int(cu[-1]), h, D) for h in (Hq, Hkv, Hkv))
+        c = torch.from_numpy(cu.astype(np.int32)).to(DEV)
+        o = K.flash_attn_varlen_func(q, k, v, c, c, max(lens), max(lens), 0.125)
+        for a, b in list(zip(cu, cu[1:]))[::9]:
+            alone = torch.tensor([0] * 65 + [b - a], dtype=torch.int32, device=DEV)
+            if b > a:
+                want = K.flash_attn_varlen_func(q[a:b], k[a:b], v[a:b], alone, alone, int(b - a), int(b - a), 0.125)
+                assert torch.equal(o[a:b], want), (a, b)
+
+
 @pytest.mark.parametrize("max_q", [(1 << 20) - 100, 1 << 20])
 def test_prefill_many_empty_workgroups(max_q):
     """Short prompts under a max_seqlen_q whose grid passes 2^20 workgroups
