@@ -240,4 +240,11 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// LDS writes of this wave visible to its other lanes (no workgroup barrier)
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace lfs

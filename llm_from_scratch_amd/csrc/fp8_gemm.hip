@@ -105,13 +105,6 @@ __device__ __forceinline__ void store_stream16(void* p, const u32x4& v) {
   asm volatile("global_store_dwordx4 %0, %1, off nt sc1" : : "v"(p), "v"(v) : "memory");
 }
 
-// LDS writes of this wave visible to its other lanes (no workgroup barrier)
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // s_waitcnt lgkmcnt(0) (LDS reads of this wave complete), vmcnt unconstrained
 __device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 

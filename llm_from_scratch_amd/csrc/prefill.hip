@@ -107,6 +107,10 @@ __device__ __forceinline__ void copy_rows(const uint8_t* base, const unsigned (&
 __device__ __forceinline__ u32x4 lds_read16(unsigned a) {
   return *(const __attribute__((address_space(3))) u32x4*)(uintptr_t)a;
 }
+__device__ __forceinline__ void lds_write8(unsigned a, uint2 v) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  *(__attribute__((address_space(3))) u32x2*)(uintptr_t)a = u32x2{v.x, v.y};
+}
 __device__ __forceinline__ uint2 lds_read_tr(unsigned a) {
   return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                                        (__attribute__((address_space(3))) v4s*)(uintptr_t)a));
@@ -264,7 +268,8 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
   const int qp = off + tq;                 // its position
   // positions of the wave's first and last row, and of the workgroup's last
   const int pfirst = __builtin_amdgcn_readfirstlane(off + (int)(min(r0 + RW * wave, rows - 1) / G));
-  const int plast = __builtin_amdgcn_readfirstlane(off + (int)(min(r0 + RW * wave + RW - 1, rows - 1) / G));
+  const int plast = r0 + RW * wave >= rows  // (-1: none, the wave only copies)
+                        ? -1 : __builtin_amdgcn_readfirstlane(off + (int)(min(r0 + RW * wave + RW - 1, rows - 1) / G));
   const int wlast = off + (int)(min(r0 + RW * NW - 1, rows - 1) / G);
   const int nkt = min(lk, wlast + 1) <= 0 ? 0 : (min(lk, wlast + 1) + KT - 1) / KT;
   const int64_t rowb = (int64_t)Hkv * RB;  // bytes per token of k / v
@@ -464,10 +469,16 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
     }
   }
 
-  // ---- normalise and store: lane l holds row l % 32, dims 32db + 8i + 4h .. +3
-  if (row < rows) {
+  // ---- normalise and store: lane l holds row l % 32, dims 32db + 8i + 4h .. +3,
+  // 16 bytes of a line per row and instruction: the rows go through LDS
+  // (swizzled as K's) and leave it with D / 8 lanes on each.  Stored from the
+  // registers, a workgroup's lines were written in pieces for 1 us at D = 128
+  // (32 / 8 heads, 64 prompts of 64: 25.6 -> 21.1 us, 65 of 128 64 -> 38, 64
+  // of 512 300 -> 255).
+  __syncthreads();  // every wave is done with the K and V tiles
+  const unsigned ob = lbase + wave * (RW * RB);
+  {
     const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-    uint16_t* dst = out + ((int64_t)(q0 + tq) * Hq + (int64_t)kh * G.d + hq) * D + 4 * h;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
@@ -475,8 +486,19 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
         uint2 w;
         w.x = pack_bf16x2(o[db][4 * x] * inv, o[db][4 * x + 1] * inv);
         w.y = pack_bf16x2(o[db][4 * x + 2] * inv, o[db][4 * x + 3] * inv);
-        *reinterpret_cast<uint2*>(dst + 32 * db + 8 * x) = w;
+        lds_write8(ob + c32 * RB + (((4 * db + x) ^ kswz<D>(c32)) << 4) + 8 * h, w);
       }
+  }
+  wave_lds_fence();
+#pragma unroll
+  for (int it = 0; it < RW / RPC; ++it) {
+    const int r = RPC * it + lane / (D / 8), c = lane % (D / 8);
+    const unsigned orow = r0 + RW * wave + r;
+    const u32x4 v = lds_read16(ob + r * RB + ((c ^ kswz<D>(r)) << 4));
+    if (orow < rows) {
+      const int t = orow / G;
+      *reinterpret_cast<u32x4*>(out + ((int64_t)(q0 + t) * Hq + (int64_t)kh * G.d + (orow - t * G.d)) * D + 8 * c) = v;
+    }
   }
 }
 
