@@ -105,7 +105,7 @@
 extern "C" {
 #endif
 
-#define LFS_ABI_VERSION 16
+#define LFS_ABI_VERSION 17
 
 /* argument errors (negative); launch errors are positive hipError_t values */
 #define LFS_EINVAL (-1)
@@ -353,6 +353,17 @@ int lfs_prefill_attention(const void* q, const void* k, const void* v, const int
                           int32_t block_size, int64_t num_slots, void* out, int64_t B,
                           int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                           int32_t max_seqlen_q, float scale, void* stream);
+
+/*
+ * The same with the longest context's length as a hint: calls of few, short
+ * tiles (max_seqlen_k to 256, no block table) run on 16-row tiles, the same
+ * bits sooner.  Without it contexts count as long.
+ */
+int lfs_prefill_attention_max_k(const void* q, const void* k, const void* v, const int32_t* cu_seqlens_q,
+                          const int32_t* cu_seqlens_k, const int32_t* block_tables, int64_t bt_stride,
+                          int32_t block_size, int64_t num_slots, void* out, int64_t B,
+                          int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                          int32_t max_seqlen_q, int32_t max_seqlen_k, float scale, void* stream);
 
 /*
  * FP8 indexer score (DSA lightning indexer):

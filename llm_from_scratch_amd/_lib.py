@@ -11,7 +11,7 @@ import ctypes
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "liblfs_kernels.so"
-ABI_VERSION = 16
+ABI_VERSION = 17
 # size of the library's static paged-decode workspace (LFS_DECODE_SCRATCH_BYTES)
 DECODE_SCRATCH_BYTES = 64 << 20
 
@@ -70,6 +70,8 @@ SIGNATURES = {
                                                _c_p, _c_p, _c_p, _c_i64, _c_p]),
     "lfs_prefill_attention": (ctypes.c_int, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i32, _c_i64, _c_p,
                                              _c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _c_f, _c_p]),
+    "lfs_prefill_attention_max_k": (ctypes.c_int, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i32, _c_i64, _c_p,
+                                                   _c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_f, _c_p]),
     "lfs_moe_align_tiles": (ctypes.c_int64, [_c_i64, _c_i32, _c_i32, _c_i32]),
     "lfs_moe_align": (ctypes.c_int, [_c_p, _c_p, _c_i64, _c_i32, _c_i32, _c_i32, _c_p, _c_p, _c_p, _c_i64, _c_p,
                                      _c_p, _c_i64, _c_p]),

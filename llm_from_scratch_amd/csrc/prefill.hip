@@ -60,6 +60,7 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef short v4s __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
 
@@ -502,6 +503,263 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
   }
 }
 
+// ---- short prompts ----
+//
+// One workgroup per (sequence, 16 query tokens, kv head), one wave per query
+// head of the group; 64-key K and V tiles go through registers into LDS, V
+// transposed, and 16x16x32 MFMAs make the same sums.  Twice the waves of the
+// kernel above at half the work each: where a call is one or few tiles long it
+// ends sooner (the softmax of 16 rows a wave against 32), and never when tiles
+// follow each other.  The rule is at prefill_short().
+constexpr int QT = 16;                // query tokens per wave (one MFMA column block)
+constexpr int NH = KT / 16;           // 16-key halves (S MFMA row blocks) per tile
+constexpr int NKS = KT / 32;          // 32-key MFMA k steps of P.V per tile
+constexpr int VT_PITCH = 2 * KT + 8;  // bytes per dim row of the transposed V tile (+ pad)
+
+template <int D, int G>
+__global__ __launch_bounds__(64 * G) void prefill_short_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k, uint16_t* __restrict__ out, int Hkv, int qtiles,
+    float scale_log2) {
+  constexpr int NDC = D / 32;                        // 32-dim chunks (MFMA k steps of S)
+  constexpr int NDB = D / 16;                        // 16-dim blocks of O^T
+  constexpr int CPK = D / 8;                         // 16-byte chunks of a key row
+  constexpr int VUN = KT / 2 * CPK;                  // (key pair, chunk) units of a V tile
+  constexpr int NT = 64 * G;                         // threads
+  constexpr int VPT = (VUN + NT - 1) / NT;           // units per thread
+  constexpr int KUN = KT * CPK;                      // 16-byte chunks of a K tile
+  constexpr int KPT = (KUN + NT - 1) / NT;           // chunks per thread
+  __shared__ __attribute__((aligned(16))) uint8_t vt[2][D * VT_PITCH];
+  __shared__ __attribute__((aligned(16))) uint8_t kt[2][KT * 2 * D];
+
+  // each XCD takes a contiguous range of (sequence, kv head) pairs, whose
+  // query tiles, last to first, share its L2
+  const int nwg = gridDim.x * gridDim.y;
+  int wid = blockIdx.y * gridDim.x + blockIdx.x;
+  if ((nwg & 7) == 0) wid = (wid & 7) * (nwg >> 3) + (wid >> 3);
+  const int pair = wid / qtiles;
+  const int i = pair / Hkv, kh = pair - i * Hkv;
+  const int tq0 = (qtiles - 1 - (wid - pair * qtiles)) * QT;  // the first query
+  const int q0 = cu_q[i], lq = cu_q[i + 1] - q0;
+  if (tq0 >= lq) return;  // the whole workgroup
+  const int k0 = cu_k[i], lk = cu_k[i + 1] - k0;
+  const int off = lk - lq;  // position of query token 0
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int h = kh * G + wave, Hq = Hkv * G;
+  const int c16 = lane & 15, g = lane >> 4;
+  const int64_t row = (int64_t)Hkv * D;  // elements per token row of k / v
+  const int64_t hoff = (int64_t)kh * D;
+
+  // keys past the context read the row of key lk - 1: their weights are 0, but
+  // their V rows still enter the product
+  auto key_elem = [&](int t) -> int64_t { return ((int64_t)k0 + min(t, lk - 1)) * row + hoff; };
+
+  // Q^T (B operand): lane l supplies query tq0 + l % 16, dims 32c + 8g .. +7
+  v8bf qb[NDC];
+  {
+    const int tq = tq0 + c16;
+#pragma unroll
+    for (int c = 0; c < NDC; ++c) {
+      uint4 w = make_uint4(0, 0, 0, 0);
+      if (tq < lq) w = *reinterpret_cast<const uint4*>(q + ((int64_t)(q0 + tq) * Hq + h) * D + c * 32 + g * 8);
+      qb[c] = __builtin_bit_cast(v8bf, w);
+    }
+  }
+  // this lane's query position; rows past lq are computed (finite) and not stored
+  const int qp = min(off + tq0 + c16, lk - 1);
+  // keys up to the last query of the tile
+  const int nkt = (max(min(lk, off + tq0 + QT), 0) + KT - 1) / KT;
+
+  // K tile in LDS: key rows of 2D bytes, 16-byte chunk c of row r at kswz
+  auto kat = [](int r, int c) -> int { return r * 2 * D + ((c ^ kswz<D>(r)) << 4); };
+  // chunk u of the tile: key u / CPK, chunk u % CPK (a row per CPK lanes)
+  auto load_k = [&](uint4 (&kr)[KPT], int t0) {
+#pragma unroll
+    for (int e = 0; e < KPT; ++e) {
+      const int u = threadIdx.x + NT * e;
+      kr[e] = make_uint4(0, 0, 0, 0);
+      if (u < KUN) kr[e] = *reinterpret_cast<const uint4*>(k + key_elem(t0 + u / CPK) + (u % CPK) * 8);
+    }
+  };
+  auto store_kt = [&](const uint4 (&kr)[KPT], int buf) {
+#pragma unroll
+    for (int e = 0; e < KPT; ++e) {
+      const int u = threadIdx.x + NT * e;
+      if (u < KUN) *reinterpret_cast<uint4*>(&kt[buf][kat(u / CPK, u % CPK)]) = kr[e];
+    }
+  };
+  // V unit u of a tile: key pair kp (keys 2kp, 2kp + 1), 16-byte chunk cc of
+  // both rows; eight consecutive units cover the chunks of one pair (whole
+  // rows per eight lanes), the pair index is swizzled by the chunk's high
+  // half so that a wave's 32-bit LDS writes below hit distinct banks
+  auto vunit = [&](int u, int& kp, int& cc) {
+    cc = (u & 7) + 8 * ((u >> 3) / (KT / 2) % (CPK / 8));
+    const int kpl = (u >> 3) % (KT / 2);
+    kp = (kpl + 8 * ((u & 7) >> 2)) % (KT / 2);
+  };
+  auto load_v = [&](uint4 (&vr)[VPT][2], int t0) {
+#pragma unroll
+    for (int e = 0; e < VPT; ++e) {
+      const int u = threadIdx.x + NT * e;
+      vr[e][0] = vr[e][1] = make_uint4(0, 0, 0, 0);
+      if (u < VUN) {
+        int kp, cc;
+        vunit(u, kp, cc);
+        vr[e][0] = *reinterpret_cast<const uint4*>(v + key_elem(t0 + 2 * kp) + cc * 8);
+        vr[e][1] = *reinterpret_cast<const uint4*>(v + key_elem(t0 + 2 * kp + 1) + cc * 8);
+      }
+    }
+  };
+  // transposed store: dim d of keys (2kp, 2kp + 1) as one 32-bit word at
+  // vt[d][2kp]
+  auto store_vt = [&](const uint4 (&vr)[VPT][2], int buf) {
+#pragma unroll
+    for (int e = 0; e < VPT; ++e) {
+      const int u = threadIdx.x + NT * e;
+      if (u < VUN) {
+        int kp, cc;
+        vunit(u, kp, cc);
+        const uint32_t* a = reinterpret_cast<const uint32_t*>(&vr[e][0]);
+        const uint32_t* b = reinterpret_cast<const uint32_t*>(&vr[e][1]);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          // dims 8cc + 2x (low halves) and 8cc + 2x + 1 (high halves)
+          const uint32_t lo = (a[x] & 0xFFFFu) | (b[x] << 16);
+          const uint32_t hi = (a[x] >> 16) | (b[x] & 0xFFFF0000u);
+          *reinterpret_cast<uint32_t*>(&vt[buf][(8 * cc + 2 * x) * VT_PITCH + kp * 4]) = lo;
+          *reinterpret_cast<uint32_t*>(&vt[buf][(8 * cc + 2 * x + 1) * VT_PITCH + kp * 4]) = hi;
+        }
+      }
+    }
+  };
+
+  v4f o[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db) o[db] = v4f{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+
+  uint4 kr[KPT], vr[VPT][2];
+  if (nkt > 0) {
+    load_k(kr, 0);
+    load_v(vr, 0);
+  }
+  for (int j = 0; j < nkt; ++j) {
+    const int t0 = j * KT;
+    const int buf = j & 1;
+    store_kt(kr, buf);
+    store_vt(vr, buf);
+    // K and V^T of tile j visible to every wave.  The buffers written next
+    // (tile j+1) were last read in tile j-1, which every wave finished
+    // before this barrier.
+    __syncthreads();
+    if (j + 1 < nkt) {
+      load_k(kr, t0 + KT);
+      load_v(vr, t0 + KT);
+    }
+    const uint8_t* kb8 = kt[buf];
+
+    // ---- S^T for the 16-key halves; the causal mask only where the tile
+    // reaches past the tile's first query position
+    const bool need_mask = t0 + KT - 1 > off + tq0;
+    float s[NH][4];
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < NH; ++kb) {
+      v4f sc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NDC; ++c) {
+        const uint4 kf = *reinterpret_cast<const uint4*>(kb8 + kat(16 * kb + c16, 4 * c + g));
+        sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, kf), qb[c], sc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[kb][r] = sc[r] * scale_log2;
+        if (need_mask && t0 + 16 * kb + 4 * g + r > qp) s[kb][r] = -INFINITY;
+        tmax = fmaxf(tmax, s[kb][r]);
+      }
+    }
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    const float m_new = fmaxf(m_run, tmax), m_exp = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = m_new == m_run ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
+    float psum = 0.f;
+    float p[NH][4];
+#pragma unroll
+    for (int kb = 0; kb < NH; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        p[kb][r] = __builtin_amdgcn_exp2f(s[kb][r] - m_exp);
+        psum += p[kb][r];
+      }
+    psum += __shfl_xor(psum, 16, 64);
+    psum += __shfl_xor(psum, 32, 64);
+    l_run = l_run * alpha + psum;
+    m_run = m_new;
+
+    // ---- O^T = O^T * alpha + V^T P^T, one MFMA k step per 32 keys
+    v8bf pb[NKS];
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        pb[ks][r] = (__bf16)p[2 * ks][r];
+        pb[ks][4 + r] = (__bf16)p[2 * ks + 1][r];
+      }
+    const uint8_t* vb = vt[buf];
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) {
+      const int dim = db * 16 + c16;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[db][r] *= alpha;
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) {
+        const uint2 lo = *reinterpret_cast<const uint2*>(vb + dim * VT_PITCH + (32 * ks + 4 * g) * 2);
+        const uint2 hi = *reinterpret_cast<const uint2*>(vb + dim * VT_PITCH + (32 * ks + 16 + 4 * g) * 2);
+        const uint4 w = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, w), pb[ks], o[db], 0, 0, 0);
+      }
+    }
+  }
+
+  // ---- normalise and store: lane l holds query tq0 + l % 16, dims 16db + 4g .. +3
+  const int tq = tq0 + c16;
+  if (tq < lq) {
+    const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+    uint16_t* dst = out + ((int64_t)(q0 + tq) * Hq + h) * D;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) {
+      uint2 w;
+      w.x = pack_bf16x2(o[db][0] * inv, o[db][1] * inv);
+      w.y = pack_bf16x2(o[db][2] * inv, o[db][3] * inv);
+      *reinterpret_cast<uint2*>(dst + db * 16 + 4 * g) = w;
+    }
+  }
+}
+
+// Whether a call goes to prefill_short_kernel: keys in token order, few and short
+// tiles.  With w = B * q heads * 16-token tiles (its waves) and t = 64-key
+// tiles of the longest context, to 256 keys: at D = 64 w * t <= 4096 (3072 from
+// t = 3; one head a group, whose workgroup is a single wave, one tile and w <=
+// 1024); at D = 128, where half as many workgroups fit a CU, w * t <= 2304 and
+// groups of 2-6 (a single wave copies too slowly, eight hold a CU's LDS).
+// us, short / long.  12 / 4 heads of 64: 1 prompt of 64 4.5 / 5.7, of 128 5.7 /
+// 6.5, of 256 8.3 / 8.5, of 384 10.8 / 10.3; 64 prompts of 64 7.1 / 7.6, 32 of
+// 128 8.9 / 8.0.  8 / 8 of 64: 1 of 64 4.9 / 5.5, 64 of 64 9.3 / 6.8.  32 / 8 of
+// 128: 1 of 64 5.4 / 6.8, 8 of 64 6.0 / 7.3, 4 of 128 7.6 / 8.7, 8 of 128 9.8 /
+// 9.6, 4 of 192 11.4 / 10.6.  8 / 8 of 128: 1 of 64 7.0 / 6.6.
+inline bool prefill_short(bool paged, int64_t B, int Hq, int G, int D, int64_t max_q, int64_t max_k) {
+  if (paged || max_k > 256 || max_q > max_k) return false;
+  const int64_t w = B * Hq * ((max_q + QT - 1) / QT), t = (max_k + KT - 1) / KT;
+  if (D == 64) return G == 1 ? w * t <= 1024 && t == 1 : w * t <= (t <= 2 ? 4096 : 3072) && (G < 8 || t <= 3);
+  return G >= 2 && G <= 6 && w * t <= 2304;
+}
+
+template <int D, int G>
+void launch_short(dim3 grid, hipStream_t st, const uint16_t* q, const uint16_t* k, const uint16_t* v,
+                  const int32_t* cu_q, const int32_t* cu_k, uint16_t* out, int Hkv, int qtiles, float sl2) {
+  hipLaunchKernelGGL((prefill_short_kernel<D, G>), grid, dim3(64 * G), 0, st, q, k, v, cu_q, cu_k, out, Hkv, qtiles, sl2);
+}
+
 }  // namespace
 }  // namespace lfs
 
@@ -512,6 +770,15 @@ extern "C" int lfs_prefill_attention(const void* q, const void* k, const void* v
                                      int64_t bt_stride, int32_t block_size, int64_t num_slots, void* out,
                                      int64_t B, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                                      int32_t max_seqlen_q, float scale, void* stream) {
+  return lfs_prefill_attention_max_k(q, k, v, cu_seqlens_q, cu_seqlens_k, block_tables, bt_stride, block_size, num_slots,
+                                     out, B, num_q_heads, num_kv_heads, head_dim, max_seqlen_q, INT32_MAX, scale, stream);
+}
+
+extern "C" int lfs_prefill_attention_max_k(const void* q, const void* k, const void* v, const int32_t* cu_seqlens_q,
+                                           const int32_t* cu_seqlens_k, const int32_t* block_tables,
+                                           int64_t bt_stride, int32_t block_size, int64_t num_slots, void* out,
+                                           int64_t B, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                           int32_t max_seqlen_q, int32_t max_seqlen_k, float scale, void* stream) {
   const int Hq = num_q_heads, Hkv = num_kv_heads, D = head_dim;
   LFS_REQUIRE(B >= 0 && Hq > 0 && Hkv > 0 && max_seqlen_q >= 0, "prefill_attention: bad shape");
   LFS_REQUIRE(D == 64 || D == 128, "prefill_attention: head_dim must be 64 or 128 (got %d)", D);
@@ -534,6 +801,23 @@ extern "C" int lfs_prefill_attention(const void* q, const void* k, const void* v
   const dim3 grid((unsigned)(wgs < kGridX ? wgs : kGridX), (unsigned)((wgs + kGridX - 1) / kGridX));
   const float sl2 = scale * 1.4426950408889634f;
   hipStream_t st = (hipStream_t)stream;
+  if (prefill_short(block_tables != nullptr, B, Hq, G, D, max_seqlen_q, max_seqlen_k)) {
+    const int qtiles = (max_seqlen_q + QT - 1) / QT;
+#define LFS_PS(DD, GG)                                                                                             \
+  case GG:                                                                                                         \
+    launch_short<DD, GG>(dim3((unsigned)(B * qtiles), (unsigned)Hkv), st, (const uint16_t*)q, (const uint16_t*)k, \
+                         (const uint16_t*)v, cu_seqlens_q, cu_seqlens_k, (uint16_t*)out, Hkv, qtiles, sl2);       \
+    break;
+    if (D == 64) {
+      switch (G) {
+        LFS_PS(64, 1) LFS_PS(64, 2) LFS_PS(64, 3) LFS_PS(64, 4) LFS_PS(64, 5) LFS_PS(64, 6) LFS_PS(64, 7) LFS_PS(64, 8)
+      }
+    } else {
+      switch (G) { LFS_PS(128, 2) LFS_PS(128, 3) LFS_PS(128, 4) LFS_PS(128, 5) LFS_PS(128, 6) }
+    }
+#undef LFS_PS
+    return check_launch("prefill_attention");
+  }
   const Div dBS = div_by(block_tables != nullptr ? block_size : 1);
 #define LFS_PF(DD, PG)                                                                                             \
   hipLaunchKernelGGL((prefill_attention_kernel<DD, PG>), grid, dim3(64 * NW), 0, st, (const uint16_t*)q,        \

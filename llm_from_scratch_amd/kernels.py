@@ -672,9 +672,10 @@ def flash_attn_varlen_func(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(D)
     o = torch.empty_like(q)
-    rc = _lib.load().lfs_prefill_attention(_ptr(q), _ptr(k), _ptr(v), _ptr(cu_seqlens_q), _ptr(cu_seqlens_k),
-                                           bt_ptr, bt_stride, BS, num_slots, _ptr(o), B, Hq, Hkv, D,
-                                           int(max_seqlen_q), float(softmax_scale), _stream(q))
+    rc = _lib.load().lfs_prefill_attention_max_k(_ptr(q), _ptr(k), _ptr(v), _ptr(cu_seqlens_q), _ptr(cu_seqlens_k),
+                                                 bt_ptr, bt_stride, BS, num_slots, _ptr(o), B, Hq, Hkv, D,
+                                                 int(max_seqlen_q), min(int(max_seqlen_k), 2 ** 31 - 1),
+                                                 float(softmax_scale), _stream(q))
     _lib.check(rc, "flash_attn_varlen_func")
     return o
 

@@ -285,6 +285,27 @@ def test_prefill_one_long_prompt_among_short(Hq, Hkv, D):
                 assert torch.equal(o[a:b], want), (a, b)
 
 
+@pytest.mark.parametrize("Hq,Hkv,D", [(3, 3, 64), (8, 4, 64), (12, 4, 64), (16, 4, 64), (5, 1, 64), (12, 2, 64),
+                                      (7, 1, 64), (16, 2, 64), (8, 4, 128), (6, 2, 128), (8, 2, 128), (10, 2, 128),
+                                      (6, 1, 128)])
+@pytest.mark.parametrize("top", [1, 16, 63, 64, 65, 129, 250])
+def test_prefill_short_prompts_same_bits(Hq, Hkv, D, top):
+    """Short whole prompts and cached prefixes in token order (16-row tiles at
+    these sizes) against the same call whose hint says that contexts are long,
+    and the oracle; every group size that the short form is compiled for."""
+    rng = np.random.default_rng(Hq * top + D)
+    lens_k = np.array([top, max(1, top - 1), 0, (top + 1) // 2, min(top, 17)])
+    lens_q = np.array([top, max(1, top // 3), 0, (top + 1) // 2, 1])
+    cu_q, cu_k = (torch.tensor(np.concatenate([[0], np.cumsum(n)]), dtype=torch.int32, device=DEV) for n in (lens_q, lens_k))
+    q = bf16(rng, int(lens_q.sum()), Hq, D)
+    k, v = (bf16(rng, int(lens_k.sum()), Hkv, D) for _ in range(2))
+    for scale in (0.125, -0.3):
+        o = K.flash_attn_varlen_func(q, k, v, cu_q, cu_k, top, top, scale)
+        assert torch.equal(o, K.flash_attn_varlen_func(q, k, v, cu_q, cu_k, top, 100000, scale))
+        ref = P.prefill_attention(f64(q), f64(k), f64(v), cu_q.cpu().numpy(), cu_k.cpu().numpy(), scale)
+        assert_close(f64(o), ref, f"short {Hq}/{Hkv} x {D}, {top}")
+
+
 @pytest.mark.parametrize("max_q", [(1 << 20) - 100, 1 << 20])
 def test_prefill_many_empty_workgroups(max_q):
     """Short prompts under a max_seqlen_q whose grid passes 2^20 workgroups
