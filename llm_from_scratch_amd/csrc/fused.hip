@@ -796,12 +796,14 @@ __device__ __forceinline__ bool all_within_60(const uint4& v) {
   return max(m[0], m[1]) <= 0x4270;  // bf16 60
 }
 
-// silu(a) for a bf16 |a| <= 60, to within about an ulp of fp32: exp(-a) as
-// exp2 of the rounded product with the rounding error put back to first
-// order, and the quotient by a reciprocal and one residual step (den lies in
-// [1, 2^87], so nothing scales or overflows).  Rounded to bf16 it equals
-// a / (1 + expf(-a)) for every such a (a test goes through all of them), at
-// some 17 instructions against 31.
+// silu(a) for a bf16 |a| <= 60: exp(-a) as exp2 of the rounded product with
+// that rounding put back to first order, and the quotient by a reciprocal and
+// one residual step (den lies in [1, 2^87], so nothing scales or overflows).
+// What is not put back is the error of the constant, log2(e) to fp32 (1.34e-8
+// relative): for negative gates the result is off by |a| times that, up to 12
+// ulp (8e-7) near -57, 2 at -10.  No bound of ulps makes the bf16 roundings
+// equal to those of a / (1 + expf(-a)); they are for every such a because a
+// test goes through all of them.  Some 17 instructions against 31.
 __device__ __forceinline__ float silu_within_60(float a) {
   const float t = a * -1.44269504f;  // -log2(e)
   const float lo = fmaf(a, -1.44269504f, -t), e = __builtin_amdgcn_exp2f(t);

@@ -45,9 +45,11 @@
 // registers and its 32-bit LDS writes out.  Bound: at D = 128 the MFMAs are
 // busy 45 % of the cycles and the VALU 55 % (the clock falls to 1.9 GHz under
 // the load), at D = 64 the VALU 75 %: exp2 takes 8 cycles a wave, and
-// max, fma, sum and rounding 2.5-5 each, per score.  Measured: six prompts of
-// 700-6000 tokens, half of each cached (GQA 32 / 8, D 128, paged): 1757 ->
-// 575 us, 296 -> 900 TFLOP/s; 16 x 2048 tokens (12 / 4, D 64): 257 -> 165 us.
+// max, fma, sum and rounding 2.5-5 each, per score.  Measured in turn on one
+// card against a 16-row tile form (a wave per head, V transposed through
+// registers): six prompts of 700-6000 tokens, half of each cached (GQA 32 / 8,
+// D 128, paged): 1870 -> 568 us, 278 -> 914 TFLOP/s; 16 x 2048 tokens (12 / 4,
+// D 64): 259 -> 149 us.  Short prompts keep that form (below).
 // Not faster: 8 waves, 32-key tiles at three waves per SIMD, the next tile's
 // scores computed beside this tile's weights, deeper operand reads, the sum
 // on the MFMAs or v_dot2 (which does not overlap the MFMAs).
@@ -87,16 +89,12 @@ __device__ __forceinline__ void copy_rows(const uint8_t* base, const unsigned (&
   rsrc[3] = 0x00020000;
   const unsigned dst = __builtin_amdgcn_readfirstlane(lds);
   unsigned keep;
-  if constexpr (N == 1) {
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\t"
-                 "s_mov_b32 m0, %0"
-                 : "=&s"(keep) : "s"(dst), "v"(off[0]), "s"(rsrc) : "memory");
-  } else if constexpr (N == 2) {
+  if constexpr (N == 2) {
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, 0 offen lds\n\t"
                  "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, 0 offen lds\n\ts_mov_b32 m0, %0"
                  : "=&s"(keep) : "s"(dst), "v"(off[0]), "v"(off[1]), "s"(rsrc) : "memory", "scc");
   } else {
-    static_assert(N == 4, "copies per wave");
+    static_assert(N == 4, "2 or 4 copies per wave");
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %6, 0 offen lds\n\t"
                  "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %6, 0 offen lds\n\t"
                  "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 %4, %6, 0 offen lds\n\t"

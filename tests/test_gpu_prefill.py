@@ -131,12 +131,11 @@ def test_prefill_long_prompt_and_graph_grid():
 
 
 @pytest.mark.parametrize("B,L,Hq,Hkv,D", [(8, 1024, 16, 8, 64), (16, 2048, 12, 4, 64)])
-def test_prefill_large_grid_subtiles_vs_torch_fp32(B, L, Hq, Hkv, D):
-    """Grids large enough for two (8 x 1024 tokens, G = 2) or four (16 x 2048
-    tokens, G = 3: the bench shape) 16-query sub-tiles per workgroup (G * 2
-    or G * 4 waves sharing each K / V tile): against causal attention
-    computed per sequence in float32 with torch on the GPU (the float64
-    oracle is too slow at this size)."""
+def test_prefill_large_grid_vs_torch_fp32(B, L, Hq, Hkv, D):
+    """Grids of several workgroups per CU, tiles of 128 (query token, head)
+    rows that begin within a token's heads or not (G = 2; G = 3: the bench
+    shape): against causal attention computed per sequence in float32 with
+    torch on the GPU (the float64 oracle is too slow at this size)."""
     g = torch.Generator(device=DEV).manual_seed(13)
     q = torch.randn(B * L, Hq, D, generator=g, device=DEV).to(torch.bfloat16)
     k = torch.randn(B * L, Hkv, D, generator=g, device=DEV).to(torch.bfloat16)
@@ -172,10 +171,10 @@ def _torch_causal_ref(qs, ks, vs, G, D, scale):
     return torch.matmul(torch.softmax(s, -1), vf).permute(1, 0, 2)
 
 
-def test_prefill_large_grid_four_subtiles_d128():
-    """Four 16-query sub-tiles per workgroup at D = 128 and G = 4 (the cfg4
-    heads, 32 / 8): 4 x 4096-token prompts fill every CU eight times with
-    64-query workgroups.  Against causal attention per sequence in float32."""
+def test_prefill_large_grid_d128():
+    """D = 128 and G = 4 (the cfg4 heads, 32 / 8): 4 x 4096-token prompts are
+    4096 workgroups of 128 rows, 16 per CU, of 1 to 64 key tiles.  Against
+    causal attention per sequence in float32."""
     B, L, Hq, Hkv, D = 4, 4096, 32, 8, 128
     g = torch.Generator(device=DEV).manual_seed(14)
     q = torch.randn(B * L, Hq, D, generator=g, device=DEV).to(torch.bfloat16)
@@ -191,10 +190,10 @@ def test_prefill_large_grid_four_subtiles_d128():
 
 
 @pytest.mark.parametrize("B,lq,cached,Hq,Hkv,D", [(16, 2048, 1536, 12, 4, 64), (8, 2048, 512, 32, 8, 128)])
-def test_prefill_large_grid_paged_cached_prefix_subtiles(B, lq, cached, Hq, Hkv, D):
+def test_prefill_large_grid_paged_cached_prefix(B, lq, cached, Hq, Hkv, D):
     """The paged kernel (a prefix-cache hit: `cached` keys already in the
-    pool) on a grid large enough for four 16-query sub-tiles per workgroup:
-    block size 256, a randomly permuted pool, -1-padded tables.  Against
+    pool) on a grid of several workgroups per CU: block size 256, a randomly
+    permuted pool, -1-padded tables.  Against
     causal attention per sequence in float32 over the gathered keys."""
     BS = 256
     lk = cached + lq
@@ -269,19 +268,20 @@ def test_prefill_ragged_work_items(Hq, Hkv, D, B, BS, scale):
 def test_prefill_one_long_prompt_among_short(Hq, Hkv, D):
     """A prompt of 2001 tokens beside 63 of 0-70 (most work items are past the
     last tile; G and Hkv of 3, 5 and 7 divide by a rounded reciprocal), a batch
-    of equal prompts, and one prompt alone: every sequence the same bits as by
-    itself in index order (beside 64 empty ones, which the search passes by)."""
+    of equal prompts, and one prompt alone (as long contexts, so that none goes
+    to the short form): every sequence the same bits as by itself in index
+    order (beside 64 empty ones, which the search passes by)."""
     rng = np.random.default_rng(Hq)
     long = [2001 if b == 40 else (7 * b) % 71 for b in range(64)]
     for lens in (long, [33] * 64, [130]):
         cu = np.concatenate([[0], np.cumsum(lens)])
         q, k, v = (bf16(rng, int(cu[-1]), h, D) for h in (Hq, Hkv, Hkv))
         c = torch.from_numpy(cu.astype(np.int32)).to(DEV)
-        o = K.flash_attn_varlen_func(q, k, v, c, c, max(lens), max(lens), 0.125)
+        o = K.flash_attn_varlen_func(q, k, v, c, c, max(lens), 100000, 0.125)
         for a, b in list(zip(cu, cu[1:]))[::9]:
             alone = torch.tensor([0] * 65 + [b - a], dtype=torch.int32, device=DEV)
             if b > a:
-                want = K.flash_attn_varlen_func(q[a:b], k[a:b], v[a:b], alone, alone, int(b - a), int(b - a), 0.125)
+                want = K.flash_attn_varlen_func(q[a:b], k[a:b], v[a:b], alone, alone, int(b - a), 100000, 0.125)
                 assert torch.equal(o[a:b], want), (a, b)
 
 
