@@ -56,6 +56,7 @@
  *                           reference names at engine/model_runner.py:291-292
  *                           (metadata :202-249; paged keys on a prefix-cache
  *                           hit, :231-237); math of model/attention/GQA.py:118-130
+ *   lfs_prefill_attention_max_k  the same with the longest context as a hint
  *   lfs_fp8_index           fp8_index(q, q_s, k, k_s), the DSA indexer score,
  *                           model/attention/utils.py:175-250 (caller
  *                           model/attention/DSA.py:105)
@@ -75,6 +76,7 @@
  *   lfs_qk_norm_rope_store  q_norm/k_norm + RoPE + KV slot write,
  *                           model/attention/GQA.py:80-95,
  *                           model/attention/utils.py:34-45
+ *   lfs_qk_norm_rope_store_kv  the same, k and v in token order as well
  *   lfs_moe_route           MoE gate, model/architecture/moe.py:45-90
  *   lfs_add_rmsnorm_route   ffn_norm + MoE gate in one launch (decode step)
  *   lfs_swiglu_quant        silu(w1 x) * w3 x, model/architecture/mlp.py:60-67,
