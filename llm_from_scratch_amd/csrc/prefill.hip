@@ -360,7 +360,12 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
   const unsigned va = lbase + 2 * TB + (4 * h + (il >> 2)) * RB +
                       (((2 * gq + ((il & 3) >> 1)) ^ vswz<D>(4 * h + (il >> 2))) << 4) + 8 * (il & 1);
 
-  float m_exp = 0.f;   // the maximum the weights are taken against (finite)
+  // The maximum the weights are taken against: 0 for a row that sees no key (a
+  // position below 0), so that it ends as 0; else the running maximum, also
+  // where that stays -infinity (every score overflowed), which makes the row
+  // NaN, as a softmax over it is.
+  const float m_none = qp < 0 ? 0.f : -INFINITY;
+  float m_exp = m_none;
   float alpha = 1.f;   // the tile's rescaling of O and of the sum
   // the causal mask, only where the tile reaches past the wave's first row;
   // then the running maximum, and O and the sum on its scale
@@ -389,7 +394,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attention_kernel(
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
       m_run = m_new;
-      m_exp = m_new == -INFINITY ? 0.f : m_new;
+      m_exp = m_new == -INFINITY ? m_none : m_new;
     }
   };
   // weights of a tile on the hardware exp2 (results below 2^-126 flush to
@@ -678,7 +683,7 @@ __global__ __launch_bounds__(64 * G) void prefill_short_kernel(
     }
     tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float m_new = fmaxf(m_run, tmax), m_exp = m_new == -INFINITY ? 0.f : m_new;
+    const float m_new = fmaxf(m_run, tmax), m_exp = m_new == -INFINITY && qp < 0 ? 0.f : m_new;
     const float alpha = m_new == m_run ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
     float psum = 0.f;
     float p[NH][4];

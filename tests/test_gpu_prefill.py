@@ -306,6 +306,24 @@ def test_prefill_short_prompts_same_bits(Hq, Hkv, D, top):
         assert_close(f64(o), ref, f"short {Hq}/{Hkv} x {D}, {top}")
 
 
+@pytest.mark.parametrize("L,D,hint", [(70, 64, 70), (70, 64, 100000), (300, 64, 300), (140, 128, 140), (140, 128, 100000)])
+def test_prefill_overflowed_rows_are_nan(L, D, hint):
+    """A row whose scores are all -infinity (products past the fp32 range) has
+    no softmax: NaN, on both tile forms; other rows, of the same token and
+    wave too, are what they are without it."""
+    rng = np.random.default_rng(L + D)
+    Hq, Hkv = 12, 4
+    q, k, v = bf16(rng, L, Hq, D), bf16(rng, L, Hkv, D).abs(), bf16(rng, L, Hkv, D)
+    cu = torch.tensor([0, L], dtype=torch.int32, device=DEV)
+    want = K.flash_attn_varlen_func(q, k, v, cu, cu, L, hint)
+    bad = torch.zeros(L, Hq, dtype=torch.bool, device=DEV)
+    for t, h in ((0, 0), (5, 7), (64, 2), (L - 1, 11)):
+        bad[t, h] = True
+    q[bad] = -3e38
+    o = K.flash_attn_varlen_func(q, k, v, cu, cu, L, hint)
+    assert bool(o[bad].isnan().all()) and torch.equal(o[~bad], want[~bad])
+
+
 @pytest.mark.parametrize("max_q", [(1 << 20) - 100, 1 << 20])
 def test_prefill_many_empty_workgroups(max_q):
     """Short prompts under a max_seqlen_q whose grid passes 2^20 workgroups
