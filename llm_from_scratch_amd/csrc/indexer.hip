@@ -20,7 +20,9 @@
 // product lose bits below 2^-149 or a sum pass 2^128 on one scale and not on
 // the other: every weight 0 or in [2^-95, 2^95) (scores are multiples of
 // 2^-18, at most 128 of them meet).  A query with any other weight -- larger,
-// smaller, infinite, NaN -- takes fmaxf and its weights unscaled.
+// smaller, infinite, NaN -- sits the walk out and is computed after it, with
+// fmaxf and its weights unscaled (a second form inside the walk cost it 1 %
+// and, at few heads, registers past an occupancy step: 8.6 -> 10.7 us).
 //
 // One workgroup per (b, 8 queries, chunk of nchunk keys), one wave per
 // query; the wave keeps its query's H/16 operand fragments in registers.
@@ -30,8 +32,6 @@
 // 16-byte chunks g and g + 4 (g = l / 16) of the 128-byte row for both q
 // and k -- the same permutation of the head dim on both sides -- so the
 // sixteen rows of one LDS read hit every bank once with the swizzle below.
-#include <type_traits>
-
 #include "common.h"
 
 namespace lfs {
@@ -66,8 +66,53 @@ __device__ __forceinline__ int kswz(int r, int c) {
   else return r * D + (c << 4);
 }
 
-template <int HB, int D>  // HB: 16-head blocks
-__global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
+// One wave's query against its workgroup's keys with fmaxf and the weights as
+// they are, 16 keys and 16 heads at a time out of memory: the same products and
+// sums.  Every index is formed again from an opaque thread id, so that the walk
+// before it holds no register for it.
+template <int HB, int D>
+__device__ __attribute__((noinline)) void index_apart(const uint8_t* __restrict__ q, const float* __restrict__ q_s,
+                                            const uint8_t* __restrict__ k, const float* __restrict__ k_s,
+                                            float* __restrict__ o, int M, int N, int H, int64_t k_stride_b,
+                                            int64_t ks_stride_b, int nchunk) {
+  unsigned tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  const int lane = tid & 63, c16 = lane & 15, g = lane >> 4;
+  const int b = blockIdx.z, m = blockIdx.y * IDX_QPW + __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n_begin = blockIdx.x * nchunk, n_end = min(N - n_begin, nchunk) + n_begin;
+  const bool lo_ok = 16 * g < D, hi_ok = 16 * (g + 4) < D;
+  const int64_t qrow = ((int64_t)b * M + m) * H;
+  auto row = [&](const uint8_t* p, bool ok) -> v8i {
+    uint4 lo = make_uint4(0, 0, 0, 0), hi = make_uint4(0, 0, 0, 0);
+    if (ok && lo_ok) lo = *reinterpret_cast<const uint4*>(p + 16 * g);
+    if (ok && hi_ok) hi = *reinterpret_cast<const uint4*>(p + 16 * (g + 4));
+    return v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+  };
+#pragma unroll 1
+  for (int n0 = n_begin; n0 < n_end; n0 += 16) {
+    const int n = n0 + c16;
+    const v8i kf = row(k + (int64_t)b * k_stride_b + (int64_t)min(n, N - 1) * D, true);
+    float acc = 0.f;
+#pragma unroll 1
+    for (int h0 = 0; h0 < 16 * HB; h0 += 16) {
+      const v4f z = {0.f, 0.f, 0.f, 0.f};
+      const v8i qf = row(q + (qrow + h0 + c16) * D, h0 + c16 < H);
+      const v4f s = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qf, kf, z, 0, 0, 0, 0, 0, 0);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int hr = h0 + 4 * g + x;
+        acc = fmaf(fmaxf(s[x], 0.f), hr < H ? q_s[qrow + hr] : 0.f, acc);
+      }
+    }
+    acc = xor_sum<32>(xor_sum<16>(acc));
+    if (g == 0 && n < n_end) o[((int64_t)b * M + m) * N + n] = acc * k_s[(int64_t)b * ks_stride_b + n];
+  }
+}
+
+// HB: 16-head blocks.  The bound keeps 128 heads of 64 at 128 registers (130
+// without: a workgroup per CU fewer, 110 -> 120 us at 2048 x 4096).
+template <int HB, int D>
+__global__ __launch_bounds__(64 * IDX_QPW, HB == 8 && D == 64 ? 4 : 1) void fp8_index_kernel(
     const uint8_t* __restrict__ q, const float* __restrict__ q_s, const uint8_t* __restrict__ k,
     const float* __restrict__ k_s, float* __restrict__ o, int M, int N, int H, int64_t k_stride_b,
     int64_t ks_stride_b, int nchunk) {
@@ -78,7 +123,7 @@ __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
   __shared__ __attribute__((aligned(16))) uint8_t kt[2][IDX_KT * D];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int b = blockIdx.z, m = blockIdx.y * IDX_QPW + wave;
-  const bool active = m < M;  // inactive waves still take part in the barriers
+  bool active = m < M;  // inactive waves still take part in the barriers
   const int n_begin = blockIdx.x * nchunk;
   const int n_end = min(N - n_begin, nchunk) + n_begin;
   const int c16 = lane & 15, g = lane >> 4;
@@ -103,15 +148,13 @@ __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int hr = hb * 16 + 4 * g + r;
-      qw[hb][r] = hr < H ? q_s[qrow + hr] : 0.f;
-      scaled = scaled && weight_scales(qw[hb][r]);
+      const float w = hr < H ? q_s[qrow + hr] : 0.f;
+      scaled = scaled && weight_scales(w);
+      qw[hb][r] = w * 0x1p12f;
     }
   }
-  scaled = __all(scaled);  // the wave's lanes hold all heads of its query
-#pragma unroll
-  for (int hb = 0; hb < HB; ++hb)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) qw[hb][r] *= scaled ? 0x1p12f : 1.f;
+  const bool apart = active && __any(!scaled);  // the wave's lanes hold all heads of its query
+  active = active && !apart;
 
   const uint8_t* kb = k + (int64_t)b * k_stride_b;
   const float* ksb = k_s + (int64_t)b * ks_stride_b;
@@ -134,38 +177,6 @@ __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
     }
   };
 
-  // the wave's scores against the tile in buffer buf, whose first key is t0
-  auto scores = [&](auto scale, int t0, int buf) {
-    constexpr bool SC = decltype(scale)::value;
-    const uint8_t* tile = kt[buf];
-#pragma unroll
-    for (int k64 = 0; k64 < IDX_KT; k64 += 64) {
-      float sum[4];
-#pragma unroll
-      for (int st = 0; st < 4; ++st) {
-        const int r = k64 + 16 * st + c16;
-        uint4 lo = make_uint4(0, 0, 0, 0), hi = make_uint4(0, 0, 0, 0);
-        if (lo_ok) lo = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g));
-        if (hi_ok) hi = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g + 4));
-        const v8i kf = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-        float acc = 0.f;
-#pragma unroll
-        for (int hb = 0; hb < HB; ++hb) {
-          const v4f z = {0.f, 0.f, 0.f, 0.f};
-          // D[head][key]: lane holds key c16, heads hb*16 + 4g .. +3
-          const v4f s = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qf[hb], kf, z, 0, 0, 0, 0, 0, 0);
-#pragma unroll
-          for (int x = 0; x < 4; ++x)
-            acc = fmaf(SC ? __builtin_amdgcn_fmed3f(s[x] * 0x1p-25f, 0.f, 1.f) : fmaxf(s[x], 0.f), qw[hb][x], acc);
-        }
-        sum[st] = acc;
-      }
-      const float tot = halve<32>(halve<16>(sum[0], sum[1]), halve<16>(sum[2], sum[3]));
-      const int n = t0 + k64 + lane;
-      if (n < n_end) orow[n] = (SC ? tot * 0x1p13f : tot) * ksb[n];
-    }
-  };
-
   const int ntiles = (n_end - n_begin + IDX_KT - 1) / IDX_KT;
   uint4 kr[CPT];
   load_tile(kr, n_begin);
@@ -176,12 +187,38 @@ __global__ __launch_bounds__(64 * IDX_QPW) void fp8_index_kernel(
     const int buf = ti & 1;
     if (ti + 1 < ntiles) load_tile(kr, t0 + IDX_KT);
     if (active) {
-      if (scaled) scores(std::true_type{}, t0, buf);
-      else scores(std::false_type{}, t0, buf);
+      const uint8_t* tile = kt[buf];
+#pragma unroll
+      for (int k64 = 0; k64 < IDX_KT; k64 += 64) {
+        float sum[4];
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+          const int r = k64 + 16 * st + c16;
+          uint4 lo = make_uint4(0, 0, 0, 0), hi = make_uint4(0, 0, 0, 0);
+          if (lo_ok) lo = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g));
+          if (hi_ok) hi = *reinterpret_cast<const uint4*>(tile + kswz<D>(r, g + 4));
+          const v8i kf = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+          float acc = 0.f;
+#pragma unroll
+          for (int hb = 0; hb < HB; ++hb) {
+            const v4f z = {0.f, 0.f, 0.f, 0.f};
+            // D[head][key]: lane holds key c16, heads hb*16 + 4g .. +3
+            const v4f s = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(qf[hb], kf, z, 0, 0, 0, 0, 0, 0);
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+              acc = fmaf(__builtin_amdgcn_fmed3f(s[x] * 0x1p-25f, 0.f, 1.f), qw[hb][x], acc);
+          }
+          sum[st] = acc;
+        }
+        const float tot = halve<32>(halve<16>(sum[0], sum[1]), halve<16>(sum[2], sum[3]));
+        const int n = t0 + k64 + lane;
+        if (n < n_end) orow[n] = (tot * 0x1p13f) * ksb[n];
+      }
     }
     if (ti + 1 < ntiles) store_tile(kr, buf ^ 1);  // buffer buf ^ 1 was last read in tile ti - 1
     __syncthreads();
   }
+  if (apart) index_apart<HB, D>(q, q_s, k, k_s, o, M, N, H, k_stride_b, ks_stride_b, nchunk);
 }
 
 }  // namespace
