@@ -30,11 +30,13 @@ namespace {
 constexpr int kAlignThreads = 1024;
 constexpr int kAlignMaxExperts = 64;
 constexpr int kTile = 128;  // rows per grouped-GEMM tile
-// Chunks whose counts one thread per expert scans, four in flight: up to here
-// it takes no longer than a wave per expert, whose exchanges cost more than
-// the round trips that they save (whole align, 3 entries a token, 9 experts:
-// 1 chunk 7.1 us against 7.6; 16 chunks 10.6 against 10.6; 18 10.1, the wave).
-constexpr int kAlignFew = 16;
+// Chunks whose counts one thread per expert scans, four in flight (fewer where
+// every expert has a wave at once): up to here it takes no longer than a wave
+// per expert, whose exchanges cost more than the round trips that they save.
+// Whole align, thread / wave, us: 9 experts 1 chunk 7.1 / 7.6, 8 10.2 / 10.3,
+// 12 10.6 / 10.2; 17 experts 12 12.9 / 12.8, 16 13.7 / 13.1; 33 experts 2
+// chunks 15.9 / 17.2, 12 17.5 / 18.0, 15 18.4 / 18.1.
+constexpr int kAlignFew = 12, kAlignFewWaves = 8;
 
 // Entry i = t * kk + j of the (token, pick) list, kk = top_k + S: picks
 // j < top_k are routed expert topk_idx[t, j] with weight topk_w[t, j]; the
@@ -112,7 +114,7 @@ __global__ __launch_bounds__(kAlignThreads) void moe_align_offsets_kernel(
   __shared__ int cnt[kAlignMaxExperts];
   __shared__ int off[kAlignMaxExperts + 1];
   const int tid = threadIdx.x, EE = E + S;
-  if (chunks <= kAlignFew) {
+  if (chunks <= (EE <= kAlignThreads / 64 ? kAlignFewWaves : kAlignFew)) {
     // one thread per expert, four chunks' counts in one round trip
     if (tid < EE) {
       int run = 0;

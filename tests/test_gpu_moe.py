@@ -277,14 +277,16 @@ def test_moe_route_nan_gate_same_weights(E, k):
         assert torch.equal(nan, got.isnan()) and torch.equal(want[~nan], got[~nan]), (e, in_bias)
 
 
-@pytest.mark.parametrize("n", [1024, 4096, 4097, 16384, 16385, 66000])
-def test_moe_align_chunk_counts(n):
-    """n entries: 1, 4, 5, 16 chunks of 1024 (a thread per expert scans their
-    counts) and 17 and 65 (a wave does), against the oracle."""
+@pytest.mark.parametrize("n,E", [(1024, 6), (4096, 6), (4097, 16), (8192, 6), (8193, 6), (66000, 6), (8193, 17),
+                                 (12288, 40), (12289, 40), (66000, 17)])
+def test_moe_align_chunk_counts(n, E):
+    """n entries: up to 8 chunks of 1024 (12 from 17 experts up), whose counts
+    a thread per expert scans, and more, where a wave does, against the
+    oracle."""
     rng = np.random.default_rng(n)
-    idx, w = rng.integers(-1, 6, (n, 1)), rng.uniform(0.05, 1.0, (n, 1)).astype(np.float32)
-    rows = K.moe_align(dev(idx), dev(w), 6)
-    token, weight, expert, entry = MO.moe_align(idx, w, 6, 0)
+    idx, w = rng.integers(-1, E, (n, 1)), rng.uniform(0.05, 1.0, (n, 1)).astype(np.float32)
+    rows = K.moe_align(dev(idx), dev(w), E)
+    token, weight, expert, entry = MO.moe_align(idx, w, E, 0)
     assert np.array_equal(rows.entry_row.cpu().numpy(), entry)
     assert np.array_equal(rows.row_token.cpu().numpy(), token)
     assert np.array_equal(rows.row_weight.cpu().numpy(), weight)
