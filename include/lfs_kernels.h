@@ -358,7 +358,7 @@ int lfs_prefill_attention(const void* q, const void* k, const void* v, const int
 
 /*
  * The same with the longest context's length as a hint: calls of few, short
- * tiles (max_seqlen_k to 256, no block table) run on 16-row tiles, the same
+ * tiles (max_seqlen_k to 256, to 64 with a block table) run on 16-row tiles, the same
  * bits sooner.  Without it contexts count as long.
  */
 int lfs_prefill_attention_max_k(const void* q, const void* k, const void* v, const int32_t* cu_seqlens_q,

@@ -519,11 +519,11 @@ constexpr int NH = KT / 16;           // 16-key halves (S MFMA row blocks) per t
 constexpr int NKS = KT / 32;          // 32-key MFMA k steps of P.V per tile
 constexpr int VT_PITCH = 2 * KT + 8;  // bytes per dim row of the transposed V tile (+ pad)
 
-template <int D, int G>
+template <int D, int G, bool PAGED>
 __global__ __launch_bounds__(64 * G) void prefill_short_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k, uint16_t* __restrict__ out, int Hkv, int qtiles,
-    float scale_log2) {
+    const int32_t* __restrict__ cu_q, const int32_t* __restrict__ cu_k, const int32_t* __restrict__ bt,
+    int64_t bt_stride, Div dBS, int64_t num_slots, uint16_t* __restrict__ out, int Hkv, int qtiles, float scale_log2) {
   constexpr int NDC = D / 32;                        // 32-dim chunks (MFMA k steps of S)
   constexpr int NDB = D / 16;                        // 16-dim blocks of O^T
   constexpr int CPK = D / 8;                         // 16-byte chunks of a key row
@@ -553,9 +553,22 @@ __global__ __launch_bounds__(64 * G) void prefill_short_kernel(
   const int64_t row = (int64_t)Hkv * D;  // elements per token row of k / v
   const int64_t hoff = (int64_t)kh * D;
 
-  // keys past the context read the row of key lk - 1: their weights are 0, but
-  // their V rows still enter the product
-  auto key_elem = [&](int t) -> int64_t { return ((int64_t)k0 + min(t, lk - 1)) * row + hoff; };
+  // Keys past the context read the row of key lk - 1: their weights are 0, but
+  // their V rows still enter the product.  Paged: one table entry per 16-key
+  // half (BS % 16 == 0); an invalid one reads slot 0.
+  auto half_slot = [&](int tstart) -> int64_t {
+    const int tc = min(tstart, lk - 1), c = (int)((unsigned)tc / dBS), BS = (int)dBS.d;
+    const int32_t blk = bt[(int64_t)i * bt_stride + min((int64_t)c, bt_stride - 1)];
+    return blk < 0 || (int64_t)blk * BS >= num_slots ? 0 : (int64_t)blk * BS + (tc - c * BS);
+  };
+  auto key_elem = [&](const int64_t (&hs)[NH], int t0, int kx) -> int64_t {  // key t0 + kx, kx < KT
+    if constexpr (PAGED) return (hs[kx >> 4] + max(0, min(kx & 15, lk - 1 - (t0 + (kx & ~15))))) * row + hoff;
+    else return ((int64_t)k0 + min(t0 + kx, lk - 1)) * row + hoff;
+  };
+  auto halves = [&](int64_t (&hs)[NH], int t0) {
+#pragma unroll
+    for (int hf = 0; hf < NH; ++hf) hs[hf] = PAGED ? half_slot(t0 + 16 * hf) : 0;
+  };
 
   // Q^T (B operand): lane l supplies query tq0 + l % 16, dims 32c + 8g .. +7
   v8bf qb[NDC];
@@ -576,12 +589,12 @@ __global__ __launch_bounds__(64 * G) void prefill_short_kernel(
   // K tile in LDS: key rows of 2D bytes, 16-byte chunk c of row r at kswz
   auto kat = [](int r, int c) -> int { return r * 2 * D + ((c ^ kswz<D>(r)) << 4); };
   // chunk u of the tile: key u / CPK, chunk u % CPK (a row per CPK lanes)
-  auto load_k = [&](uint4 (&kr)[KPT], int t0) {
+  auto load_k = [&](uint4 (&kr)[KPT], const int64_t (&hs)[NH], int t0) {
 #pragma unroll
     for (int e = 0; e < KPT; ++e) {
       const int u = threadIdx.x + NT * e;
       kr[e] = make_uint4(0, 0, 0, 0);
-      if (u < KUN) kr[e] = *reinterpret_cast<const uint4*>(k + key_elem(t0 + u / CPK) + (u % CPK) * 8);
+      if (u < KUN) kr[e] = *reinterpret_cast<const uint4*>(k + key_elem(hs, t0, u / CPK) + (u % CPK) * 8);
     }
   };
   auto store_kt = [&](const uint4 (&kr)[KPT], int buf) {
@@ -600,7 +613,7 @@ __global__ __launch_bounds__(64 * G) void prefill_short_kernel(
     const int kpl = (u >> 3) % (KT / 2);
     kp = (kpl + 8 * ((u & 7) >> 2)) % (KT / 2);
   };
-  auto load_v = [&](uint4 (&vr)[VPT][2], int t0) {
+  auto load_v = [&](uint4 (&vr)[VPT][2], const int64_t (&hs)[NH], int t0) {
 #pragma unroll
     for (int e = 0; e < VPT; ++e) {
       const int u = threadIdx.x + NT * e;
@@ -608,8 +621,8 @@ __global__ __launch_bounds__(64 * G) void prefill_short_kernel(
       if (u < VUN) {
         int kp, cc;
         vunit(u, kp, cc);
-        vr[e][0] = *reinterpret_cast<const uint4*>(v + key_elem(t0 + 2 * kp) + cc * 8);
-        vr[e][1] = *reinterpret_cast<const uint4*>(v + key_elem(t0 + 2 * kp + 1) + cc * 8);
+        vr[e][0] = *reinterpret_cast<const uint4*>(v + key_elem(hs, t0, 2 * kp) + cc * 8);
+        vr[e][1] = *reinterpret_cast<const uint4*>(v + key_elem(hs, t0, 2 * kp + 1) + cc * 8);
       }
     }
   };
@@ -642,9 +655,11 @@ __global__ __launch_bounds__(64 * G) void prefill_short_kernel(
   float m_run = -INFINITY, l_run = 0.f;
 
   uint4 kr[KPT], vr[VPT][2];
+  int64_t hs[NH];
   if (nkt > 0) {
-    load_k(kr, 0);
-    load_v(vr, 0);
+    halves(hs, 0);
+    load_k(kr, hs, 0);
+    load_v(vr, hs, 0);
   }
   for (int j = 0; j < nkt; ++j) {
     const int t0 = j * KT;
@@ -656,8 +671,9 @@ __global__ __launch_bounds__(64 * G) void prefill_short_kernel(
     // before this barrier.
     __syncthreads();
     if (j + 1 < nkt) {
-      load_k(kr, t0 + KT);
-      load_v(vr, t0 + KT);
+      halves(hs, t0 + KT);
+      load_k(kr, hs, t0 + KT);
+      load_v(vr, hs, t0 + KT);
     }
     const uint8_t* kb8 = kt[buf];
 
@@ -739,28 +755,24 @@ __global__ __launch_bounds__(64 * G) void prefill_short_kernel(
   }
 }
 
-// Whether a call goes to prefill_short_kernel: keys in token order, few and short
-// tiles.  With w = B * q heads * 16-token tiles (its waves) and t = 64-key
-// tiles of the longest context, to 256 keys: at D = 64 w * t <= 4096 (3072 from
-// t = 3; one head a group, whose workgroup is a single wave, one tile and w <=
-// 1024); at D = 128, where half as many workgroups fit a CU, w * t <= 2304 and
-// groups of 2-6 (a single wave copies too slowly, eight hold a CU's LDS).
+// Whether a call goes to prefill_short_kernel: few and short tiles.  With w = B *
+// q heads * 16-token tiles (its waves) and t = 64-key tiles of the longest
+// context, to 256 keys: at D = 64 w * t <= 4096 (3072 from t = 3; one head a
+// group, whose workgroup is a single wave, one tile and w <= 1024); at D = 128,
+// where half as many workgroups fit a CU, w * t <= 2304 and groups of 2-6 (a
+// single wave copies too slowly, eight hold a CU's LDS).  Through a block table
+// one tile only, as its look-ups come before every tile's loads (16 of 64 keys
+// 0.94 of the long form's time, 64 of 128 1.02, 64 of 256 1.06).
 // us, short / long.  12 / 4 heads of 64: 1 prompt of 64 4.5 / 5.7, of 128 5.7 /
 // 6.5, of 256 8.3 / 8.5, of 384 10.8 / 10.3; 64 prompts of 64 7.1 / 7.6, 32 of
 // 128 8.9 / 8.0.  8 / 8 of 64: 1 of 64 4.9 / 5.5, 64 of 64 9.3 / 6.8.  32 / 8 of
 // 128: 1 of 64 5.4 / 6.8, 8 of 64 6.0 / 7.3, 4 of 128 7.6 / 8.7, 8 of 128 9.8 /
 // 9.6, 4 of 192 11.4 / 10.6.  8 / 8 of 128: 1 of 64 7.0 / 6.6.
 inline bool prefill_short(bool paged, int64_t B, int Hq, int G, int D, int64_t max_q, int64_t max_k) {
-  if (paged || max_k > 256 || max_q > max_k) return false;
+  if (max_k > (paged ? KT : 256) || max_q > max_k) return false;
   const int64_t w = B * Hq * ((max_q + QT - 1) / QT), t = (max_k + KT - 1) / KT;
   if (D == 64) return G == 1 ? w * t <= 1024 && t == 1 : w * t <= (t <= 2 ? 4096 : 3072) && (G < 8 || t <= 3);
   return G >= 2 && G <= 6 && w * t <= 2304;
-}
-
-template <int D, int G>
-void launch_short(dim3 grid, hipStream_t st, const uint16_t* q, const uint16_t* k, const uint16_t* v,
-                  const int32_t* cu_q, const int32_t* cu_k, uint16_t* out, int Hkv, int qtiles, float sl2) {
-  hipLaunchKernelGGL((prefill_short_kernel<D, G>), grid, dim3(64 * G), 0, st, q, k, v, cu_q, cu_k, out, Hkv, qtiles, sl2);
 }
 
 }  // namespace
@@ -806,10 +818,15 @@ extern "C" int lfs_prefill_attention_max_k(const void* q, const void* k, const v
   hipStream_t st = (hipStream_t)stream;
   if (prefill_short(block_tables != nullptr, B, Hq, G, D, max_seqlen_q, max_seqlen_k)) {
     const int qtiles = (max_seqlen_q + QT - 1) / QT;
+    const dim3 sgrid((unsigned)(B * qtiles), (unsigned)Hkv);
+#define LFS_PSP(DD, GG, PG)                                                                                        \
+  hipLaunchKernelGGL((prefill_short_kernel<DD, GG, PG>), sgrid, dim3(64 * GG), 0, st, (const uint16_t*)q,         \
+                     (const uint16_t*)k, (const uint16_t*)v, cu_seqlens_q, cu_seqlens_k, block_tables, bt_stride, \
+                     div_by(PG ? block_size : 1), num_slots, (uint16_t*)out, Hkv, qtiles, sl2)
 #define LFS_PS(DD, GG)                                                                                             \
   case GG:                                                                                                         \
-    launch_short<DD, GG>(dim3((unsigned)(B * qtiles), (unsigned)Hkv), st, (const uint16_t*)q, (const uint16_t*)k, \
-                         (const uint16_t*)v, cu_seqlens_q, cu_seqlens_k, (uint16_t*)out, Hkv, qtiles, sl2);       \
+    if (block_tables != nullptr) LFS_PSP(DD, GG, true);                                                            \
+    else LFS_PSP(DD, GG, false);                                                                                   \
     break;
     if (D == 64) {
       switch (G) {
@@ -819,6 +836,7 @@ extern "C" int lfs_prefill_attention_max_k(const void* q, const void* k, const v
       switch (G) { LFS_PS(128, 2) LFS_PS(128, 3) LFS_PS(128, 4) LFS_PS(128, 5) LFS_PS(128, 6) }
     }
 #undef LFS_PS
+#undef LFS_PSP
     return check_launch("prefill_attention");
   }
   const Div dBS = div_by(block_tables != nullptr ? block_size : 1);

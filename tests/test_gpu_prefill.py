@@ -306,6 +306,39 @@ def test_prefill_short_prompts_same_bits(Hq, Hkv, D, top):
         assert_close(f64(o), ref, f"short {Hq}/{Hkv} x {D}, {top}")
 
 
+@pytest.mark.parametrize("Hq,Hkv,D", [(12, 4, 64), (8, 8, 64), (8, 1, 64), (32, 8, 128), (6, 1, 128)])
+@pytest.mark.parametrize("BS", [16, 48])
+def test_prefill_short_paged_same_bits(Hq, Hkv, D, BS):
+    """Contexts of one 64-key tile through a block table (16-row tiles at these
+    sizes), with cached prefixes, an entry out of range and a pool that holds
+    NaN past every context: the long form's bits, and the oracle."""
+    rng = np.random.default_rng(Hq + D + BS)
+    lens_k, lens_q = np.array([64, 17, 33, 0, 48, 1]), np.array([64, 1, 20, 0, 16, 1])
+    cu_q, cu_k = (torch.tensor(np.concatenate([[0], np.cumsum(n)]), dtype=torch.int32, device=DEV) for n in (lens_q, lens_k))
+    nblk = -(-lens_k // BS)
+    perm = rng.permutation(np.arange(1, int(nblk.sum()) + 3))
+    bt = np.full((len(lens_k), int(nblk.max()) + 1), -1, np.int32)
+    at = 0
+    for b, n in enumerate(nblk):
+        bt[b, :n] = perm[at:at + n]
+        at += n
+    q = bf16(rng, int(lens_q.sum()), Hq, D)
+    k, v = (bf16(rng, len(perm) + 1, BS, Hkv, D) for _ in range(2))
+    for pool in (k, v):
+        for b, n in enumerate(lens_k):
+            if n % BS:
+                pool[int(bt[b, n // BS]), int(n % BS):] = float("nan")
+    args = (q, k, v, cu_q, cu_k)
+    o = K.flash_attn_varlen_func(*args, 64, 64, 0.125, block_table=torch.from_numpy(bt).to(DEV))
+    assert torch.equal(o, K.flash_attn_varlen_func(*args, 64, 9999, 0.125, block_table=torch.from_numpy(bt).to(DEV)))
+    ref = P.prefill_attention(f64(q), np.nan_to_num(f64(k)), np.nan_to_num(f64(v)), cu_q.cpu().numpy(), cu_k.cpu().numpy(),
+                              0.125, block_tables=bt)
+    assert_close(f64(o), ref, f"short paged {Hq}/{Hkv} x {D}, blocks of {BS}")
+    bt[0, 0] = len(perm) + 7  # out of range: slot 0, on both forms
+    o, long = (K.flash_attn_varlen_func(*args, 64, m, 0.125, block_table=torch.from_numpy(bt).to(DEV)) for m in (64, 9999))
+    assert torch.equal(o, long)
+
+
 @pytest.mark.parametrize("L,D,hint", [(70, 64, 70), (70, 64, 100000), (300, 64, 300), (140, 128, 140), (140, 128, 100000)])
 def test_prefill_overflowed_rows_are_nan(L, D, hint):
     """A row whose scores are all -infinity (products past the fp32 range) has
