@@ -29,6 +29,7 @@ stream; outputs are allocated here, as the reference wrappers do
 from __future__ import annotations
 
 import math
+import numbers
 from typing import Optional, Tuple
 
 import torch
@@ -643,7 +644,8 @@ def flash_attn_varlen_func(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     sequence i is row cu_seqlens_k[i] + t); with it (int32 [B, max_blocks],
     a prefix-cache hit) they are the paged caches [num_blocks, block_size,
     Hkv, D].  Queries of sequence i sit at the last lq positions of its lk
-    keys and attend to keys up to their own position.  softmax_scale
+    keys and attend to keys up to their own position.  max_seqlen_k chooses the
+    tiles and never the result: any value is taken.  softmax_scale
     defaults to 1/sqrt(D).  Returns bf16 [total_q, Hq, D]."""
     assert causal, "only causal prefill attention is provided"
     assert q.dim() == 3 and q.is_contiguous(), "q must be contiguous [total_q, Hq, D]"
@@ -671,11 +673,13 @@ def flash_attn_varlen_func(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     assert Dk == D, "head_dim mismatch between q and k"
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(D)
+    # a hint only: whatever is not a whole number (None, a device scalar, whose
+    # value would take a synchronisation) counts as "long"
+    max_k = max(-1, min(int(max_seqlen_k), 2 ** 31 - 1)) if isinstance(max_seqlen_k, numbers.Integral) else 2 ** 31 - 1
     o = torch.empty_like(q)
     rc = _lib.load().lfs_prefill_attention_max_k(_ptr(q), _ptr(k), _ptr(v), _ptr(cu_seqlens_q), _ptr(cu_seqlens_k),
                                                  bt_ptr, bt_stride, BS, num_slots, _ptr(o), B, Hq, Hkv, D,
-                                                 int(max_seqlen_q), min(int(max_seqlen_k), 2 ** 31 - 1),
-                                                 float(softmax_scale), _stream(q))
+                                                 int(max_seqlen_q), max_k, float(softmax_scale), _stream(q))
     _lib.check(rc, "flash_attn_varlen_func")
     return o
 

@@ -339,6 +339,27 @@ def test_prefill_short_paged_same_bits(Hq, Hkv, D, BS):
     assert torch.equal(o, long)
 
 
+def test_prefill_any_max_seqlen_k():
+    """max_seqlen_k is a hint: absent, not a whole number, on the device (not
+    read, so that the call can be captured), too small, negative or past 32
+    bits, the result is the same."""
+    rng = np.random.default_rng(5)
+    cu = torch.tensor([0, 90, 91, 200], dtype=torch.int32, device=DEV)
+    q, k, v = bf16(rng, 200, 12, 64), bf16(rng, 200, 4, 64), bf16(rng, 200, 4, 64)
+    want = K.flash_attn_varlen_func(q, k, v, cu, cu, 109, 109)
+    on_gpu = (cu[1:] - cu[:-1]).max()
+    for m in (None, float("inf"), np.int64(109), 109.0, torch.tensor(109), on_gpu, 1, 0, -1, -2 ** 40, 2 ** 40):
+        assert torch.equal(K.flash_attn_varlen_func(q, k, v, cu, cu, 109, m), want), str(m)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        o = K.flash_attn_varlen_func(q, k, v, cu, cu, 109, on_gpu)
+    for _ in range(3):
+        o.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, want)
+
+
 @pytest.mark.parametrize("L,D,hint", [(70, 64, 70), (70, 64, 100000), (300, 64, 300), (140, 128, 140), (140, 128, 100000)])
 def test_prefill_overflowed_rows_are_nan(L, D, hint):
     """A row whose scores are all -infinity (products past the fp32 range) has
